@@ -94,7 +94,6 @@ void launch_q8_retile(hipStream_t s, const uint8_t* blocks, int n, int k, uint8_
 enum { PF_EPI_STORE = 0, PF_EPI_RESID = 1, PF_EPI_SWIGLU = 2, PF_EPI_BIAS = 3, PF_EPI_BIAS_GELU = 4,
        PF_EPI_BIAS_SILU = 5, PF_EPI_BIAS_RESID = 6 };
 int pf_max_context();  // positions the prefill attention supports
-hipError_t prepare_kernels_pf();
 // RMSNorm(src) * gain (hidden 1024) -> q8_0 codes / scales; normed_out (nullable)
 void launch_pf_norm_quant(hipStream_t s, const float* src, int S, const float* gain, float eps, int8_t* codes,
                           float* scales, float* normed_out);

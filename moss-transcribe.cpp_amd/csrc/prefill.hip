@@ -13,22 +13,18 @@
 //                    add / SwiGLU
 //   k_pf_quant       q8_0 conversion of f32 rows (the SwiGLU output)
 //   k_pf_qk_rope     q/k RMSNorm + NEOX RoPE, K/V written into the cache
-//   k_pf_attn_mma    causal attention on f32 MFMA, 16 query rows of one q
-//                    head per wave over the cache, in two passes over the
-//                    64-key chunks, writing the o-projection's q8_0 activation
+//   k_attn_block     causal attention on f32 MFMA (attn_block.hpp), writing the
+//                    o-projection's q8_0 activation
 // Every reduction follows the canonical order of device_common.hpp, so hidden
 // rows and the KV cache equal the verify path's and the oracle's bit for bit:
 //   * GEMM: per output, 4 K-slices of block pairs, even / odd fma chains per
 //     slice in block order, ((s0 + s1) + s2) + s3 per parity, then even + odd;
-//   * attention: pass 1 takes every chunk's column maxima m_c (exact in any
-//     order) and M = max m_c; pass 2 recomputes the scores, p = exp(w - m_c),
-//     l_c = butterfly sum, O_c = fma chain over the chunk's keys, and merges in
-//     chunk order, L = fma(l_c, f_c, L), O = fma(O_c, f_c, O), f_c = exp(m_c - M)
-//     -- the same fma chains the verify path's merge runs, without storing the
-//     per-chunk partials.
+//   * attention: attn_block.hpp, the same chunk terms and merge chain the verify
+//     path runs.
 #include <hip/hip_fp16.h>
 #include <hip/hip_runtime.h>
 
+#include "attn_block.hpp"
 #include "device_common.hpp"
 
 namespace mtg {
@@ -357,315 +353,10 @@ k_pf_qk_rope(const float* __restrict__ qkv, int S, int past0, int n_heads, int n
   }
 }
 
-// ------------------------------------------------------------ attention ----
-// grid (n_heads / kPfHeads, ceil(S / kPfRows)): a workgroup takes query rows
-// r0 .. r0 + kPfRows - 1 (positions past0 + r0 + t) of the kPfHeads q heads of
-// one kv head; the blocks with the most chunks are numbered first. Keys
-// 0 .. past0 + r0 + kPfRows - 1 come from the cache (this block's rows were
-// appended by k_pf_qk_rope). The output rows leave as the o-projection's q8_0
-// activation: codes [S][n_heads * 128], scales [S][n_heads * 4].
-constexpr int kPfHeads = 2;     // q heads per workgroup (one kv head's group)
-constexpr int kPfRowTiles = 2;  // query rows per workgroup / 16
-constexpr int kPfRows = 16 * kPfRowTiles;
-
-// ------------------------------------------------ attention on f32 MFMA ----
-// k_pf_attn_mma: the causal attention of k_pf_attn with the chunk softmax kept in
-// registers. Workgroup = the two q heads of one kv head x 32 query rows; wave w
-// owns the 16 rows r0 + 16 (w & 1) + j (j = lane % 16) of q head hq0 + w / 2.
-//   scores: key tile t (16 keys) is one chain of 32 MFMAs over head_dim,
-//     A = K rows, B = the wave's q rows (registers). Row i of the A operand is
-//     key 16 t + 4 (i % 4) + i / 4, so output register r of lane (g, j)
-//     (g = lane / 16) holds key 16 t + 4 r + g: the B operand of P.V MFMA
-//     m = 4 t + r (keys 4 m .. 4 m + 3 in order) with no data movement.
-//   chunk max and sum: in-lane over t and r, then across lanes xor 32, 16 (the
-//     sum in the butterfly's pairing: key levels 32, 16, 8, 4 in the lane, 2, 1
-//     across lanes).
-//   P.V: head_dim tile dt (16) is one chain of 16 MFMAs over the chunk's keys,
-//     A = V^T.
-// The chunks go through LDS: K rows at slot 16 t + 4 g + r for key 16 t + 4 r + g,
-// element 4 s + g at g * 32 + s; V^T rows d with key 4 m + g at g * 16 + m. Pass 1
-// (row maxima) double-buffers K in the two regions; pass 2 holds K in one and
-// V^T in the other, the next chunk's loads in flight during the arithmetic.
-// A wave skips the chunks that lie wholly after its last row (their terms are
-// exact zeros of the merge).
-constexpr int kPaKs = kHeadDim + 4;              // K slab row stride (floats)
-constexpr int kPaVs = 64 + 4;                    // V^T slab row stride
-constexpr int kPaRegion = kHeadDim * kPaVs;      // floats per region (>= 64 * kPaKs)
-constexpr size_t kPaLds = (size_t)2 * kPaRegion * 4;
-static_assert(64 * kPaKs <= kPaRegion, "K slab fits a region");
-
-// this thread's share of a chunk of K (keys key0 ..): key tid / 4, elements
-// 32 (tid % 4) .. + 31; of V: keys 4 (4 mq + x) + g (x < 4), elements 8 u .. 8 u + 7
-// with (g, mq, u) = (tid / 64, tid / 16 % 4, tid % 16). Rows past kvlen read row
-// kvlen - 1 and are zeroed at the store.
-template <int KVH>
-struct PaRegs {
-  v4f r[8];
-};
-template <int KVH>
-__device__ __forceinline__ void pa_load_k(const uint8_t* kh, int key0, int kvlen, PaRegs<KVH>& R) {
-  constexpr int es = KVH ? 2 : 4;
-  const int tid = threadIdx.x, key = min(key0 + (tid >> 2), kvlen - 1), q = tid & 3;
-  const uint8_t* src = kh + ((size_t)key * kHeadDim + 32 * q) * es;
-  if constexpr (KVH) {
-#pragma unroll
-    for (int x = 0; x < 4; ++x) {
-      const v4i h = *(const v4i*)(src + 16 * x);  // 8 halves: elements 32 q + 8 x ..
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        R.r[2 * x + e / 2][2 * (e % 2)] = half_bits_to_float((uint16_t)((uint32_t)h[e] & 0xffff));
-        R.r[2 * x + e / 2][2 * (e % 2) + 1] = half_bits_to_float((uint16_t)((uint32_t)h[e] >> 16));
-      }
-    }
-  } else {
-#pragma unroll
-    for (int x = 0; x < 8; ++x) R.r[x] = *(const v4f*)(src + 16 * x);
-  }
-}
-template <int KVH>
-__device__ __forceinline__ void pa_store_k(float* s, int key0, int kvlen, const PaRegs<KVH>& R) {
-  const int tid = threadIdx.x, key = tid >> 2, q = tid & 3;
-  const int slot = (key & ~15) | ((key & 3) << 2) | ((key >> 2) & 3);
-  const bool live = key0 + key < kvlen;
-  // R.r[x][e] is element 32 q + 4 x + e = 4 s + g with s = 8 q + x, g = e
-#pragma unroll
-  for (int e = 0; e < 4; ++e)
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      v4f o;
-#pragma unroll
-      for (int x = 0; x < 4; ++x) o[x] = live ? R.r[4 * h + x][e] : 0.0f;
-      *(v4f*)(s + slot * kPaKs + e * 32 + 8 * q + 4 * h) = o;
-    }
-}
-template <int KVH>
-__device__ __forceinline__ void pa_load_v(const uint8_t* vh, int key0, int kvlen, PaRegs<KVH>& R) {
-  constexpr int es = KVH ? 2 : 4;
-  const int tid = threadIdx.x, u = tid & 15, mq = (tid >> 4) & 3, g = tid >> 6;
-#pragma unroll
-  for (int x = 0; x < 4; ++x) {
-    const int key = min(key0 + 4 * (4 * mq + x) + g, kvlen - 1);
-    const uint8_t* src = vh + ((size_t)key * kHeadDim + 8 * u) * es;
-    if constexpr (KVH) {
-      const v4i h = *(const v4i*)src;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        R.r[2 * x + e / 2][2 * (e % 2)] = half_bits_to_float((uint16_t)((uint32_t)h[e] & 0xffff));
-        R.r[2 * x + e / 2][2 * (e % 2) + 1] = half_bits_to_float((uint16_t)((uint32_t)h[e] >> 16));
-      }
-    } else {
-      R.r[2 * x] = *(const v4f*)src;
-      R.r[2 * x + 1] = *(const v4f*)(src + 16);
-    }
-  }
-}
-template <int KVH>
-__device__ __forceinline__ void pa_store_v(float* s, int key0, int kvlen, const PaRegs<KVH>& R) {
-  const int tid = threadIdx.x, u = tid & 15, mq = (tid >> 4) & 3, g = tid >> 6;
-  // R.r[2 x + e / 4][e % 4] is element 8 u + e of key 4 (4 mq + x) + g
-#pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    v4f o;
-#pragma unroll
-    for (int x = 0; x < 4; ++x) o[x] = key0 + 4 * (4 * mq + x) + g < kvlen ? R.r[2 * x + e / 4][e % 4] : 0.0f;
-    *(v4f*)(s + (8 * u + e) * kPaVs + g * 16 + 4 * mq) = o;
-  }
-}
-
-template <int KVH, bool OUTF>
-__global__ void __launch_bounds__(256, 2)
-k_pf_attn_mma(const float* __restrict__ q, int n_heads, int n_kv_heads, KvLayer kv, int past0, int S,
-              int8_t* __restrict__ ocodes, float* __restrict__ oscales, float* __restrict__ ofl) {
-  extern __shared__ v4f pa_lds_v4[];
-  float* reg0 = (float*)pa_lds_v4;
-  float* reg1 = reg0 + kPaRegion;
-  const int hq0 = blockIdx.x * kPfHeads, g_kv = hq0 / (n_heads / n_kv_heads);
-  const int r0 = (gridDim.y - 1 - blockIdx.y) * kPfRows;  // the blocks with the most chunks start first
-  const int kvlen = past0 + S;
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, j = lane & 15, g = lane >> 4;
-  const int hq = hq0 + (wave >> 1), rw = r0 + 16 * (wave & 1);  // this wave's head and first row
-  const int row = rw + j;
-  const int nch = min(past0 + r0 + kPfRows - 1, kvlen - 1) / kChunk + 1;  // the workgroup's chunks
-  const int wlast = min(past0 + rw + 15, kvlen - 1);                    // this wave's last key
-  constexpr int es = KVH ? 2 : 4;
-  const uint8_t* kh = (const uint8_t*)kv.k + (size_t)g_kv * kv.max_seq * kHeadDim * es;
-  const uint8_t* vh = (const uint8_t*)kv.v + (size_t)g_kv * kv.max_seq * kHeadDim * es;
-  const float scale = __fdiv_rn(1.0f, dev_sqrtf((float)kHeadDim));
-  // B operand of the scores: q[row][4 s + g] (f16-rounded for an f16 cache)
-  float qb[32];
-  {
-    const float* qr = q + ((size_t)min(row, S - 1) * n_heads + hq) * kHeadDim + g;
-#pragma unroll
-    for (int s = 0; s < 32; ++s) {
-      const float v = row < S ? qr[4 * s] : 0.0f;
-      qb[s] = KVH ? f16_round(v) : v;
-    }
-  }
-  const int pos = past0 + row;  // this row's last key
-  auto scores = [&](const float* sk, int key0, float (&w)[4][4]) {
-    v4f acc[4];
-#pragma unroll
-    for (int t = 0; t < 4; ++t) acc[t] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-    for (int x = 0; x < 8; ++x) {
-      v4f a[4];
-#pragma unroll
-      for (int t = 0; t < 4; ++t) a[t] = *(const v4f*)(sk + (16 * t + j) * kPaKs + g * 32 + 4 * x);
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-#pragma unroll
-        for (int t = 0; t < 4; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[t][e], qb[4 * x + e], acc[t], 0, 0, 0);
-    }
-#pragma unroll
-    for (int t = 0; t < 4; ++t)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int key = key0 + 16 * t + 4 * r + g;
-        w[t][r] = (row < S && key <= pos) ? __fmul_rn(acc[t][r], scale) : -INFINITY;
-      }
-  };
-  PaRegs<KVH> R;
-  // pass 1: row maxima over all chunks; K double-buffered in the two regions
-  pa_load_k<KVH>(kh, 0, kvlen, R);
-  pa_store_k<KVH>(reg0, 0, kvlen, R);
-  __syncthreads();
-  float M = -INFINITY;
-  for (int c = 0; c < nch; ++c) {
-    const bool last = c + 1 == nch;
-    pa_load_k<KVH>(kh, last ? 0 : 64 * (c + 1), kvlen, R);  // pass 2 starts again at chunk 0
-    if (64 * c <= wlast) {
-      float w[4][4];
-      scores((c & 1) ? reg1 : reg0, 64 * c, w);
-#pragma unroll
-      for (int t = 0; t < 4; ++t)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) M = fmaxf(M, w[t][r]);
-    }
-    pa_store_k<KVH>(((c + 1) & 1) ? reg1 : reg0, last ? 0 : 64 * (c + 1), kvlen, R);
-    __syncthreads();
-  }
-  M = pair_max_f<32>(M);
-  M = pair_max_f<16>(M);
-  // pass 2: K of chunk 0 sits in region nch & 1; V^T goes to the other region
-  float* sk = (nch & 1) ? reg1 : reg0;
-  float* sv = (nch & 1) ? reg0 : reg1;
-  pa_load_v<KVH>(vh, 0, kvlen, R);
-  pa_store_v<KVH>(sv, 0, kvlen, R);
-  __syncthreads();
-  float L = 0.0f;
-  v4f O[8];
-#pragma unroll
-  for (int dt = 0; dt < 8; ++dt) O[dt] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-  for (int c = 0; c < nch; ++c) {
-    const bool more = c + 1 < nch, live = 64 * c <= wlast;
-    if (more) pa_load_k<KVH>(kh, 64 * (c + 1), kvlen, R);
-    float p[4][4];
-    float mc = -INFINITY, lc = 0.0f;
-    if (live) {
-      float w[4][4];
-      scores(sk, 64 * c, w);
-#pragma unroll
-      for (int t = 0; t < 4; ++t)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) mc = fmaxf(mc, w[t][r]);
-      mc = pair_max_f<32>(mc);
-      mc = pair_max_f<16>(mc);
-#pragma unroll
-      for (int t = 0; t < 4; ++t)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          float pv = (mc == -INFINITY || w[t][r] == -INFINITY) ? 0.0f : dev_expf(__fsub_rn(w[t][r], mc));
-          p[t][r] = KVH ? f16_round(pv) : pv;
-        }
-      float u[2][4], x4[4];
-#pragma unroll
-      for (int t = 0; t < 2; ++t)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) u[t][r] = __fadd_rn(p[t][r], p[t + 2][r]);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) x4[r] = __fadd_rn(u[0][r], u[1][r]);
-      lc = pair_add_f<32>(__fadd_rn(__fadd_rn(x4[0], x4[2]), __fadd_rn(x4[1], x4[3])));
-      lc = pair_add_f<16>(lc);
-    }
-    __syncthreads();  // K of chunk c is consumed
-    if (more) {
-      pa_store_k<KVH>(sk, 64 * (c + 1), kvlen, R);
-      pa_load_v<KVH>(vh, 64 * (c + 1), kvlen, R);
-    }
-    if (live) {
-      v4f oc[8];
-#pragma unroll
-      for (int dt = 0; dt < 8; ++dt) oc[dt] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-      for (int x = 0; x < 4; ++x) {
-        v4f av[8];
-#pragma unroll
-        for (int dt = 0; dt < 8; ++dt) av[dt] = *(const v4f*)(sv + (16 * dt + j) * kPaVs + g * 16 + 4 * x);
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-#pragma unroll
-          for (int dt = 0; dt < 8; ++dt)
-            oc[dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[dt][e], p[x][e], oc[dt], 0, 0, 0);
-      }
-      const float f = mc == -INFINITY ? 0.0f : dev_expf(__fsub_rn(mc, M));
-      L = fmaf(lc, f, L);
-#pragma unroll
-      for (int dt = 0; dt < 8; ++dt)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) O[dt][r] = fmaf(oc[dt][r], f, O[dt][r]);
-    }
-    __syncthreads();  // V^T of chunk c is consumed, K of chunk c + 1 is staged
-    if (more) pa_store_v<KVH>(sv, 64 * (c + 1), kvlen, R);
-  }
-  // O[dt][r]: element 16 dt + 4 g + r of row `row`
-  const int QN = n_heads * kHeadDim;
-  float o[8][4];
-#pragma unroll
-  for (int dt = 0; dt < 8; ++dt)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) o[dt][r] = __fdiv_rn(O[dt][r], L);
-  if constexpr (OUTF) {
-    if (row < S) {
-      float* orow = ofl + (size_t)row * QN + hq * kHeadDim + 4 * g;
-#pragma unroll
-      for (int dt = 0; dt < 8; ++dt) *(v4f*)(orow + 16 * dt) = v4f{o[dt][0], o[dt][1], o[dt][2], o[dt][3]};
-    }
-  } else {
-    // q8_0 block b = elements 32 b .. 32 b + 31 = tiles 2 b, 2 b + 1 over the four lane groups
-#pragma unroll
-    for (int b = 0; b < 4; ++b) {
-      uint32_t u = 0;
-#pragma unroll
-      for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) u = max(u, __float_as_uint(fabsf(o[2 * b + h][r])));
-      u = pair_max_u<32>(u);
-      u = pair_max_u<16>(u);
-      const float amax = __uint_as_float(u);
-      const float id = amax != 0.0f ? __fdiv_rn(127.0f, amax) : 0.0f;
-      if (row < S) {
-        const size_t rowoff = (size_t)row * QN + hq * kHeadDim;
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          uint32_t word = 0;
-#pragma unroll
-          for (int r = 0; r < 4; ++r)
-            word |= (uint32_t)(uint8_t)(int8_t)rintf(__fmul_rn(o[2 * b + h][r], id)) << (8 * r);
-          *(uint32_t*)(ocodes + rowoff + 16 * (2 * b + h) + 4 * g) = word;
-        }
-        if (g == 0)
-          oscales[(size_t)row * (QN / 32) + (hq * kHeadDim) / 32 + b] =
-              __half2float(__float2half_rn(__fdiv_rn(amax, 127.0f)));
-      }
-    }
-  }
-}
-
 }  // namespace
 
 // ================================================================ launches ==
-// The buffer descriptors of the attention cover a kv head's rows with a 32-bit
-// byte count.
+// A kv head's rows in 32-bit byte offsets.
 int pf_max_context() { return (int)(0x7fffffffu / (kHeadDim * 4)); }
 
 void launch_pf_norm_quant(hipStream_t s, const float* src, int S, const float* gain, float eps, int8_t* codes,
@@ -704,28 +395,32 @@ void launch_pf_qk_rope(hipStream_t s, const float* qkv, int S, int past0, int n_
 
 void launch_pf_attn(hipStream_t s, const float* q, int n_heads, int n_kv_heads, KvLayer kv, int past0, int S,
                     int8_t* ocodes, float* oscales, float* ofl) {
-  const dim3 grid((unsigned)(n_heads / kPfHeads), (unsigned)((S + kPfRows - 1) / kPfRows));
-#define MTG_PF_ATTN(KVH, OUTF)                                                                                \
-  hipLaunchKernelGGL((k_pf_attn_mma<KVH, OUTF>), grid, dim3(256), kPaLds, s, q, n_heads, n_kv_heads, kv, past0, S, \
-                     ocodes, oscales, ofl)
+  const int es = kv.f16 ? 2 : 4;
+  AttnBlockArgs a{};
+  a.q = q;
+  a.k = (const uint8_t*)kv.k;
+  a.v = (const uint8_t*)kv.v;
+  a.head_bytes = (size_t)kv.max_seq * kHeadDim * es;
+  a.key_bytes = kHeadDim * es;
+  a.q_stride = n_heads * kHeadDim;
+  a.group = n_heads / n_kv_heads;
+  a.past = past0;
+  a.S = S;
+  a.kvlen = past0 + S;
+  a.out = ofl;
+  a.ocodes = ocodes;
+  a.oscales = oscales;
+  const dim3 grid((unsigned)(n_heads / 2), (unsigned)((S + 15) / 16));
+#define MTG_PF_ATTN(KVH, OUTQ) \
+  hipLaunchKernelGGL((k_attn_block<kHeadDim, KVH, true, OUTQ>), grid, dim3(256), AbLds<kHeadDim>::bytes, s, a)
   if (ofl) {
-    if (kv.f16) MTG_PF_ATTN(1, true);
-    else MTG_PF_ATTN(0, true);
-  } else {
     if (kv.f16) MTG_PF_ATTN(1, false);
     else MTG_PF_ATTN(0, false);
+  } else {
+    if (kv.f16) MTG_PF_ATTN(1, true);
+    else MTG_PF_ATTN(0, true);
   }
 #undef MTG_PF_ATTN
-}
-
-hipError_t prepare_kernels_pf() {
-  const void* fns[] = {(const void*)k_pf_attn_mma<0, false>, (const void*)k_pf_attn_mma<1, false>,
-                       (const void*)k_pf_attn_mma<0, true>, (const void*)k_pf_attn_mma<1, true>};
-  for (const void* f : fns) {
-    const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kPaLds);
-    if (e != hipSuccess) return e;
-  }
-  return hipSuccess;
 }
 
 }  // namespace mtg
