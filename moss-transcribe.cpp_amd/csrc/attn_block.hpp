@@ -24,7 +24,8 @@
 // Measured against two exact passes with K and V^T staged by the whole workgroup:
 // 1,600 rows, f32 cache 289 -> 200 us per layer (the MFMAs alone: 69 us; the rest is
 // the estimates' reads of K at the start, vector work and the uneven causal blocks);
-// 2,048 rows after 14,336, f16 cache 3.84 -> 2.6 ms (1.64 ms).
+// 2,048 rows after 14,336, f16 cache 3.84 -> 2.6 ms (1.64 ms); the
+// encoder's 1,500 rows x 16 heads 202 -> 161 us (60 us).
 #pragma once
 
 #include <hip/hip_fp16.h>

@@ -10,10 +10,8 @@
 //              lane partials, butterfly) -> q8_0 codes for the next GEMM;
 //              q / k / v / out / fc1 / fc2 on the block GEMM of the prefill
 //              (q8_0 weights x q8_0 activations, int8 MFMA) with bias, GELU or
-//              residual epilogues; k_enc_attn_mma: bidirectional attention
-//              on f32 MFMA, 16 query rows of one head per wave over all rows
-//              in 64-key chunks (two passes: row maxima, then exp / sums /
-//              context merged in chunk order)
+//              residual epilogues; k_attn_block (attn_block.hpp): bidirectional
+//              attention on f32 MFMA, 32 query rows of one head per workgroup
 //   adaptor    merge consecutive rows (a view), fc1 + SiLU, fc2, LayerNorm
 // Every reduction keeps the oracle's order (oracle/oracle.cpp, encoder
 // section), so results equal it bit for bit.
@@ -28,6 +26,7 @@
 #include <string>
 #include <vector>
 
+#include "attn_block.hpp"
 #include "device_common.hpp"
 #include "mtg_internal.hpp"
 
@@ -36,7 +35,6 @@ namespace {
 using namespace dev;
 
 constexpr int kEncHd = 64;      // head_dim
-constexpr int kEncRows = 64;    // query rows per attention workgroup (16 per wave)
 constexpr int kEncMaxChunks = 32;  // rows <= 2048
 constexpr int kConvTile = 64;   // outputs per conv workgroup: 64 rows x 64 channels
 constexpr int kConvIcb = 16;    // input channels staged per step
@@ -215,212 +213,6 @@ k_enc_ln(const float* __restrict__ src, int S, const float* __restrict__ w, cons
   }
 }
 
-// ------------------------------------------------------------ attention ----
-// Bidirectional attention on f32 MFMA (v_mfma_f32_16x16x4f32, whose 4-term dot
-// is the sequential fma chain fma(a3, b3, fma(a2, b2, fma(a1, b1, fma(a0, b0, c))))).
-// Workgroup = head blockIdx.x, rows r0 .. r0 + 63; wave w owns the 16 query rows
-// r0 + 16 w + j (j = lane % 16) over all keys, in 64-key chunks staged in LDS by
-// the whole workgroup (double-buffered, the next chunk's loads in flight during
-// the current chunk's arithmetic).
-//   scores: key tile t (16 keys) is one MFMA chain over head_dim, A = K rows,
-//     B = this wave's q rows (registers). A row i of tile t is key
-//     16 t + 4 (i % 4) + i / 4, so the output register r of lane (g, j)
-//     (g = lane / 16) holds the score of key 16 t + 4 r + g: key 4 m + g with
-//     m = 4 t + r, which is where the P.V MFMA m (keys 4 m .. 4 m + 3, in order)
-//     wants its B operand. The probabilities never leave the registers.
-//   chunk sum: the xor butterfly over the chunk's keys: levels 32 and 16 (t),
-//     8 and 4 (r) inside the lane, 2 and 1 (g) across lanes xor 32 and 16.
-//   P.V: head_dim tile dt is one MFMA chain over the chunk's keys, A = V^T.
-// Pass 1 takes each row's maximum over all keys; pass 2 recomputes the scores,
-// the chunk maxima m_c, p = exp(w - m_c), l_c and O_c, and merges the chunks in
-// order with f = exp(m_c - M): L = fma(l_c, f, L), O = fma(O_c, f, O).
-// LDS: K rows at slot 16 t + 4 g + r for key 16 t + 4 r + g, element 4 s + kk at
-// kk * 16 + s; V^T rows d with key 4 m + g at g * 16 + m. Rows 68 floats apart.
-constexpr int kEaStride = 68;
-constexpr int kEaBuf = 64 * kEaStride;  // floats per staged chunk (K or V^T)
-constexpr size_t kEaLds = (size_t)4 * kEaBuf * 4;  // K and V^T, two buffers each
-
-__device__ __forceinline__ void ea_load_k(const float* __restrict__ k, int key0, int T, int W, int h, v4f (&r)[4]) {
-  const int tid = threadIdx.x, key = tid >> 2, q = tid & 3;
-  const float* src = k + (size_t)min(key0 + key, T - 1) * W + h * kEncHd + 16 * q;
-#pragma unroll
-  for (int x = 0; x < 4; ++x) r[x] = *(const v4f*)(src + 4 * x);
-}
-// K row key (element 16 q + 4 x + e = 4 s + kk with s = 4 q + x, kk = e) to slot
-// 16 t + 4 g + r of key 16 t + 4 r + g; rows past T are zero
-__device__ __forceinline__ void ea_store_k(float* s_k, int key0, int T, const v4f (&r)[4]) {
-  const int tid = threadIdx.x, key = tid >> 2, q = tid & 3;
-  const int slot = (key & ~15) | ((key & 3) << 2) | ((key >> 2) & 3);
-  const bool live = key0 + key < T;
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    v4f o;
-#pragma unroll
-    for (int x = 0; x < 4; ++x) o[x] = live ? r[x][e] : 0.0f;
-    *(v4f*)(s_k + slot * kEaStride + e * 16 + 4 * q) = o;
-  }
-}
-// V: thread (g, mq, u) loads keys 4 (4 mq + x) + g, elements 4 u .. 4 u + 3
-__device__ __forceinline__ void ea_load_v(const float* __restrict__ v, int key0, int T, int W, int h, v4f (&r)[4]) {
-  const int tid = threadIdx.x, u = tid & 15, mq = (tid >> 4) & 3, g = tid >> 6;
-#pragma unroll
-  for (int x = 0; x < 4; ++x) {
-    const int key = 4 * (4 * mq + x) + g;
-    r[x] = *(const v4f*)(v + (size_t)min(key0 + key, T - 1) * W + h * kEncHd + 4 * u);
-  }
-}
-__device__ __forceinline__ void ea_store_v(float* s_v, int key0, int T, const v4f (&r)[4]) {
-  const int tid = threadIdx.x, u = tid & 15, mq = (tid >> 4) & 3, g = tid >> 6;
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    v4f o;
-#pragma unroll
-    for (int x = 0; x < 4; ++x) o[x] = key0 + 4 * (4 * mq + x) + g < T ? r[x][e] : 0.0f;
-    *(v4f*)(s_v + (4 * u + e) * kEaStride + g * 16 + 4 * mq) = o;
-  }
-}
-
-__global__ void __launch_bounds__(256, 2)
-k_enc_attn_mma(const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v, int T, int W,
-               float* __restrict__ out) {
-  extern __shared__ v4f ea_lds_v4[];
-  float* s_k = (float*)ea_lds_v4;  // [2][kEaBuf]
-  float* s_v = s_k + 2 * kEaBuf;   // [2][kEaBuf]
-  const int h = blockIdx.x, r0 = blockIdx.y * kEncRows;
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, j = lane & 15, g = lane >> 4;
-  const int nch = (T + 63) / 64;
-  const float scale = __fdiv_rn(1.0f, dev_sqrtf((float)kEncHd));
-  // the B operand of the scores: q[row][4 s + g], s < 16 (rows past T: zeros)
-  const int row = r0 + 16 * wave + j;
-  float qb[16];
-  {
-    const float* qr = q + (size_t)min(row, T - 1) * W + h * kEncHd + g;
-#pragma unroll
-    for (int s = 0; s < 16; ++s) qb[s] = row < T ? qr[4 * s] : 0.0f;
-  }
-  // scores of the staged chunk at key0: w[t][r] = key 16 t + 4 r + g, row j
-  auto scores = [&](const float* sk, int key0, float (&w)[4][4]) {
-    v4f acc[4];
-    v4f a[4][4];
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      acc[t] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-      const float* kr = sk + (16 * t + j) * kEaStride + g * 16;
-#pragma unroll
-      for (int x = 0; x < 4; ++x) a[t][x] = *(const v4f*)(kr + 4 * x);
-    }
-#pragma unroll
-    for (int s = 0; s < 16; ++s)
-#pragma unroll
-      for (int t = 0; t < 4; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[t][s >> 2][s & 3], qb[s], acc[t], 0, 0, 0);
-#pragma unroll
-    for (int t = 0; t < 4; ++t)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) w[t][r] = key0 + 16 * t + 4 * r + g < T ? __fmul_rn(acc[t][r], scale) : -INFINITY;
-  };
-  v4f kr[4], vr[4];
-  // chunk n of the whole walk: n < nch is pass 1 (K only), n >= nch pass 2 (K and V)
-  ea_load_k(k, 0, T, W, h, kr);
-  ea_store_k(s_k, 0, T, kr);
-  __syncthreads();
-  float M = -INFINITY;
-  for (int n = 0; n < nch; ++n) {
-    const int nx = n + 1 < nch ? n + 1 : 0;  // the next staged chunk (pass 2 starts at chunk 0)
-    ea_load_k(k, 64 * nx, T, W, h, kr);
-    if (n + 1 == nch) ea_load_v(v, 0, T, W, h, vr);
-    float w[4][4];
-    scores(s_k + (n & 1) * kEaBuf, 64 * n, w);
-#pragma unroll
-    for (int t = 0; t < 4; ++t)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) M = fmaxf(M, w[t][r]);
-    ea_store_k(s_k + ((n + 1) & 1) * kEaBuf, 64 * nx, T, kr);
-    if (n + 1 == nch) ea_store_v(s_v + ((n + 1) & 1) * kEaBuf, 0, T, vr);
-    __syncthreads();
-  }
-  M = pair_max_f<32>(M);
-  M = pair_max_f<16>(M);
-  float L = 0.0f;
-  v4f O[4];
-#pragma unroll
-  for (int dt = 0; dt < 4; ++dt) O[dt] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-  for (int c = 0; c < nch; ++c) {
-    const int b = (nch + c) & 1;
-    const bool more = c + 1 < nch;
-    if (more) {
-      ea_load_k(k, 64 * (c + 1), T, W, h, kr);
-      ea_load_v(v, 64 * (c + 1), T, W, h, vr);
-    }
-    float w[4][4];
-    scores(s_k + b * kEaBuf, 64 * c, w);
-    float mc = -INFINITY;
-#pragma unroll
-    for (int t = 0; t < 4; ++t)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) mc = fmaxf(mc, w[t][r]);
-    mc = pair_max_f<32>(mc);
-    mc = pair_max_f<16>(mc);
-    float p[4][4];
-#pragma unroll
-    for (int t = 0; t < 4; ++t)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) p[t][r] = w[t][r] == -INFINITY ? 0.0f : dev_expf(__fsub_rn(w[t][r], mc));
-    // l_c: key levels 32, 16 (t), 8, 4 (r) in the lane, 2, 1 (g) across lanes
-    float lc;
-    {
-      float u[2][4];
-#pragma unroll
-      for (int t = 0; t < 2; ++t)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) u[t][r] = __fadd_rn(p[t][r], p[t + 2][r]);
-      float x[4];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) x[r] = __fadd_rn(u[0][r], u[1][r]);
-      const float y0 = __fadd_rn(x[0], x[2]), y1 = __fadd_rn(x[1], x[3]);
-      lc = pair_add_f<32>(__fadd_rn(y0, y1));
-      lc = pair_add_f<16>(lc);
-    }
-    // O_c: head_dim tiles dt, A = V^T rows 16 dt + j, B = p (key 4 m + g at p[m / 4][m % 4])
-    const float* sv = s_v + b * kEaBuf;
-    v4f oc[4];
-    v4f av[4][4];
-#pragma unroll
-    for (int dt = 0; dt < 4; ++dt) {
-      oc[dt] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-      const float* vrow = sv + (16 * dt + j) * kEaStride + g * 16;
-#pragma unroll
-      for (int x = 0; x < 4; ++x) av[dt][x] = *(const v4f*)(vrow + 4 * x);
-    }
-#pragma unroll
-    for (int m = 0; m < 16; ++m)
-#pragma unroll
-      for (int dt = 0; dt < 4; ++dt)
-        oc[dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[dt][m >> 2][m & 3], p[m >> 2][m & 3], oc[dt], 0, 0, 0);
-    const float f = dev_expf(__fsub_rn(mc, M));
-    L = fmaf(lc, f, L);
-#pragma unroll
-    for (int dt = 0; dt < 4; ++dt)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) O[dt][r] = fmaf(oc[dt][r], f, O[dt][r]);
-    if (more) {
-      ea_store_k(s_k + (b ^ 1) * kEaBuf, 64 * (c + 1), T, kr);
-      ea_store_v(s_v + (b ^ 1) * kEaBuf, 64 * (c + 1), T, vr);
-    }
-    __syncthreads();
-  }
-  // O[dt][r] is element 16 dt + 4 g + r of row j
-  if (row < T) {
-    float* orow = out + (size_t)row * W + h * kEncHd + 4 * g;
-#pragma unroll
-    for (int dt = 0; dt < 4; ++dt) {
-      v4f o4;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) o4[r] = __fdiv_rn(O[dt][r], L);
-      *(v4f*)(orow + 16 * dt) = o4;
-    }
-  }
-}
-
 size_t q8_tiles_bytes(int n, int k) { return (size_t)(n / 16) * (k / kPairK) * kUnitBytes; }
 
 }  // namespace
@@ -583,10 +375,6 @@ int mtg_encoder_create(const mtg_encoder_desc* d, mtg_encoder** out) {
   int rc = e->check(hipStreamCreateWithFlags(&e->stream, hipStreamNonBlocking), "stream");
   if (!rc) rc = e->check(hipEventCreate(&e->ev0), "event");
   if (!rc) rc = e->check(hipEventCreate(&e->ev1), "event");
-  if (!rc)
-    rc = e->check(hipFuncSetAttribute((const void*)k_enc_attn_mma, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                      (int)kEaLds),
-                  "attention LDS");
   // staging for the raw q8_0 rows of the largest matrix
   size_t raw_max = (size_t)std::max(F, std::max(D, H)) * (std::max(F, IN) / 32) * 34;
   uint8_t* staging = rc ? nullptr : (uint8_t*)e->dalloc(raw_max);
@@ -690,13 +478,22 @@ int mtg_encoder_encode(mtg_encoder* e, const float* mel, float* out, int32_t* ro
                      e->conv1_w, e->conv1_b, e->mel, M, NF, D, (const float*)nullptr, e->c1);
   hipLaunchKernelGGL((k_enc_conv_mma<2, false>), dim3((R + kConvTile - 1) / kConvTile, D / kConvTile), dim3(256), 0, s,
                      e->conv2_w, e->conv2_b, e->c1, D, NF, D, e->pos, e->x);
-  const dim3 agrid((unsigned)hp.n_heads, (unsigned)((R + kEncRows - 1) / kEncRows));
+  const dim3 agrid((unsigned)hp.n_heads, (unsigned)((R + 31) / 32));
+  AttnBlockArgs attn{};
+  attn.q = e->q;
+  attn.k = (const uint8_t*)e->k;
+  attn.v = (const uint8_t*)e->v;
+  attn.head_bytes = kEncHd * 4;
+  attn.key_bytes = D * 4;
+  attn.q_stride = D;
+  attn.S = attn.kvlen = R;
+  attn.out = e->a;
   for (const mtg_encoder::Layer& L : e->layers) {
     e->ln(e->x, R, L.attn_ln_w, L.attn_ln_b, 1e-5f, true, nullptr);
     e->gemm(PF_EPI_BIAS, L.q_w, D, D, R, e->q, L.q_b);
     e->gemm(PF_EPI_STORE, L.k_w, D, D, R, e->k, nullptr);
     e->gemm(PF_EPI_BIAS, L.v_w, D, D, R, e->v, L.v_b);
-    hipLaunchKernelGGL(k_enc_attn_mma, agrid, dim3(256), kEaLds, s, e->q, e->k, e->v, R, D, e->a);
+    hipLaunchKernelGGL((k_attn_block<kEncHd, 0, false, false>), agrid, dim3(256), AbLds<kEncHd>::bytes, s, attn);
     e->quant(e->a, R, D);
     e->gemm(PF_EPI_BIAS_RESID, L.o_w, D, D, R, e->x, L.o_b);
     e->ln(e->x, R, L.ffn_ln_w, L.ffn_ln_b, 1e-5f, true, nullptr);
