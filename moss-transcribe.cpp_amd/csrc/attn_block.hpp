@@ -48,7 +48,7 @@ struct AttnBlockArgs {
   int group;            // q heads per kv head (causal)
   int past, S, kvlen;   // rows 0 .. S - 1 at positions past + row; kvlen keys
   float* out;           // f32 rows [row][q_stride], or
-  int8_t* ocodes;       // q8_0 codes [row][q_stride] and scales [row][q_stride / 32]
+  int8_t* ocodes;       // q8_0 codes and scales of rows of q_stride (q8_rows_code, q8_rows_scale)
   float* oscales;
 };
 
@@ -571,9 +571,9 @@ __global__ void __launch_bounds__(256, 2) k_attn_block(const AttnBlockArgs A) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) word[i] |= (uint32_t)(uint8_t)(int8_t)rintf(__fmul_rn(o[h][4 * i + e], id)) << (8 * e);
       }
-      const size_t at = (size_t)orow * A.q_stride + ooff + (KVH ? 32 * g + 16 * h : 64 * h + 16 * g);
-      *(uint4*)(A.ocodes + at) = make_uint4(word[0], word[1], word[2], word[3]);
-      if (KVH ? h == 0 : (g & 1) == 0) A.oscales[at / 32] = __half2float(__float2half_rn(__fdiv_rn(amax, 127.0f)));
+      const int at = ooff + (KVH ? 32 * g + 16 * h : 64 * h + 16 * g);
+      *(uint4*)(A.ocodes + q8_rows_code(A.S, orow, at / 16)) = make_uint4(word[0], word[1], word[2], word[3]);
+      if (KVH ? h == 0 : (g & 1) == 0) A.oscales[q8_rows_scale(A.S, orow, at / 32)] = __half2float(__float2half_rn(__fdiv_rn(amax, 127.0f)));
     }
   } else {
     if (orow >= A.S) return;

@@ -154,6 +154,16 @@ __device__ __forceinline__ float half_bits_to_float(uint16_t h) {
   return __half2float(__ushort_as_half(h));
 }
 
+// The q8_0 activation of S rows for the block GEMM, in the order its MFMA reads it.
+// Codes: 64-element steps of 64-row blocks, each [4 parts of 16 elements][64 rows][16
+// bytes]; byte offset of elements 16 k16 .. of a row. Scales: [32-block][rows padded to 64].
+__device__ __forceinline__ size_t q8_rows_code(int S, int row, int k16) {
+  return (((size_t)(k16 >> 2) * ((S + 63) >> 6) + (row >> 6)) * 256 + (k16 & 3) * 64 + (row & 63)) * 16;
+}
+__device__ __forceinline__ size_t q8_rows_scale(int S, int row, int block) {
+  return (size_t)block * (((S + 63) >> 6) << 6) + row;
+}
+
 // ------------------------------------------------------ lane exchanges ---
 // lane_xor<O>(v): the value of lane (lane ^ O) of a 64-lane wave, with VALU
 // lane moves instead of LDS permutes: DPP quad_perm (O = 1, 2), two bank-masked

@@ -208,8 +208,8 @@ k_enc_ln(const float* __restrict__ src, int S, const float* __restrict__ w, cons
       for (int q = 0; q < 4; ++q) u |= (uint32_t)(uint8_t)(int8_t)rintf(__fmul_rn(y[4 * w4 + q], id)) << (8 * q);
       packed[w4] = u;
     }
-    *(uint4*)(codes + (size_t)row * D + 16 * lane) = make_uint4(packed[0], packed[1], packed[2], packed[3]);
-    if ((lane & 1) == 0) scales[(size_t)row * (D / 32) + lane / 2] = __half2float(__float2half_rn(d));
+    *(uint4*)(codes + q8_rows_code(S, row, lane)) = make_uint4(packed[0], packed[1], packed[2], packed[3]);
+    if ((lane & 1) == 0) scales[q8_rows_scale(S, row, lane / 2)] = __half2float(__float2half_rn(d));
   }
 }
 
@@ -428,7 +428,8 @@ int mtg_encoder_create(const mtg_encoder_desc* d, mtg_encoder** out) {
     e->h1 = (float*)e->dalloc((size_t)N * H * 4);
     e->h2 = (float*)e->dalloc((size_t)N * H * 4);
     e->ad_out = (float*)e->dalloc((size_t)N * H * 4);
-    const size_t KC = std::max((size_t)R * std::max(F, D), (size_t)N * IN);
+    // whole 64-row blocks (q8_rows_code)
+    const size_t KC = std::max((size_t)((R + 63) / 64 * 64) * std::max(F, D), (size_t)((N + 63) / 64 * 64) * IN);
     e->codes = (int8_t*)e->dalloc(KC);
     e->scales = (float*)e->dalloc(KC / 32 * 4);
     if (wt == MTG_TYPE_F16) {

@@ -5,11 +5,10 @@
 // The verify path processes at most 16 rows per weight pass; a 1,600-row prompt
 // through it costs 100 full weight streams. Here every layer is a short
 // sequence of kernels over all rows of a block (up to kPfRows):
-//   k_pf_norm_quant  RMSNorm * gain and the q8_0 activation conversion, compact
-//                    layout: codes [S][K] int8, scales [S][K/32] (f16 values)
-//   k_pf_gemm        q8_0 weight tiles x activation rows on v_mfma_i32_16x16x64_i8
-//                    (block-diagonal B operand from LDS-staged codes: two exact
-//                    per-block int32 dots per MFMA), epilogue store / residual
+//   k_pf_norm_quant  RMSNorm * gain and the q8_0 activation conversion, codes and
+//                    scales (f16 values) in the GEMM's order (q8_rows_code)
+//   k_pf_gemm        q8_0 weight tiles x activation rows on v_mfma_i32_32x32x32_i8
+//                    (one exact int32 dot per block), epilogue store / residual
 //                    add / SwiGLU
 //   k_pf_quant       q8_0 conversion of f32 rows (the SwiGLU output)
 //   k_pf_qk_rope     q/k RMSNorm + NEOX RoPE, K/V written into the cache
@@ -80,8 +79,8 @@ k_pf_norm_quant(const float* __restrict__ src, int S, const float* __restrict__ 
     for (int b = 0; b < 4; ++b) u |= (uint32_t)(uint8_t)(int8_t)rintf(__fmul_rn(y[4 * w4 + b], id)) << (8 * b);
     packed[w4] = u;
   }
-  *(uint4*)(codes + (size_t)row * kH + 16 * lane) = make_uint4(packed[0], packed[1], packed[2], packed[3]);
-  if ((lane & 1) == 0) scales[(size_t)row * (kH / 32) + lane / 2] = __half2float(__float2half_rn(d));
+  *(uint4*)(codes + q8_rows_code(S, row, lane)) = make_uint4(packed[0], packed[1], packed[2], packed[3]);
+  if ((lane & 1) == 0) scales[q8_rows_scale(S, row, lane / 2)] = __half2float(__float2half_rn(d));
 }
 
 // q8_0 conversion of f32 rows of K (a multiple of 32): one wave per row, lane =
@@ -114,194 +113,167 @@ k_pf_quant(const float* __restrict__ src, int S, int K, int8_t* __restrict__ cod
       for (int e = 0; e < 4; ++e) u |= (uint32_t)(uint8_t)(int8_t)rintf(__fmul_rn(v[4 * w4 + e], id)) << (8 * e);
       packed[w4] = u;
     }
-    uint4* dst = (uint4*)(codes + (size_t)row * K + 32 * b);
-    dst[0] = make_uint4(packed[0], packed[1], packed[2], packed[3]);
-    dst[1] = make_uint4(packed[4], packed[5], packed[6], packed[7]);
-    scales[(size_t)row * (K / 32) + b] = __half2float(__float2half_rn(d));
+    *(uint4*)(codes + q8_rows_code(S, row, 2 * b)) = make_uint4(packed[0], packed[1], packed[2], packed[3]);
+    *(uint4*)(codes + q8_rows_code(S, row, 2 * b + 1)) = make_uint4(packed[4], packed[5], packed[6], packed[7]);
+    scales[q8_rows_scale(S, row, b)] = __half2float(__float2half_rn(d));
   }
 }
 
 // ----------------------------------------------------------------- GEMM ----
-// out[s][n] for the 64 weight rows of blockIdx.x (wave w: tile 4 blockIdx.x + w;
-// for SwiGLU waves 0, 1 take gate tiles 2 blockIdx.x + {0, 1} and waves 2, 3 the
-// same tiles of the up matrix, meeting in LDS for the epilogue) and the 64
-// activation rows of blockIdx.y (8 column groups of 8). The block pairs run in
-// order; per pair the activation codes of the 64 rows are staged in LDS (the
-// next pair's already in flight in registers), and each wave's B operand of
-// column group cg holds 16 code bytes of row 8 cg + j % 8, block 2 bp + j / 8,
-// when (lane / 16) / 2 == j / 8 (j = lane % 16), else zeros, so each MFMA returns
-// the exact int32 dot of every (weight row, activation row, block). The K-slices
-// run one after the other, so one accumulator per slice and a running total
-// give ((s0 + s1) + s2) + s3 per parity, then even + odd.
+// out[s][n] = the canonical q8_0 dot of weight row n and activation row s: per
+// 32-block the exact int32 sum (v_mfma_i32_32x32x32_i8), then one fma of it with
+// dw * dx (exact in f32) into the even or odd chain of the K-slice; slices add
+// ((s0 + s1) + s2) + s3 per parity, then even + odd.
+//
+// What bounds it: those float steps. Every output needs a conversion, a product
+// and an fma per block, 48 vector instructions per 32 x 32 block of outputs (196
+// cycles with the MFMA's 35 beside them), 61 us per decoder layer at 1,600 rows. So
+// a wave keeps a 32 x 32 tile's running sums in registers and nothing else is vector
+// work: both operands lie in memory in the order the MFMA takes them and go straight
+// to LDS, several 64-element steps ahead of their use. A workgroup takes 64 activation
+// rows x 64 weight rows (SwiGLU: 32 of gate and the same 32 of up).
 enum { PF_STORE = 0, PF_RESID = 1, PF_SWIGLU = 2, PF_BIAS = 3, PF_BIAS_GELU = 4, PF_BIAS_SILU = 5, PF_BIAS_RESID = 6 };
-constexpr int kPfRowBytes = 80;  // LDS stride of a staged 64-byte code row (bank spread)
+typedef int v16i __attribute__((ext_vector_type(16)));
 
-template <int EPI>
-__global__ void __launch_bounds__(256)
+// 16 (4) bytes per lane from memory to LDS at lds + 16 (4) * lane, counted in vmcnt.
+// lds is a byte address, uniform over the wave.
+__device__ __forceinline__ void lds_fill16(const void* src, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(lds) : "memory");
+}
+__device__ __forceinline__ void lds_fill4(const void* src, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(src), "s"(lds) : "memory");
+}
+
+// One 64-element step in LDS: the codes of 4 weight units, then 4 parts x 64 rows x 16
+// bytes of the activation, the units' scales (4 x 32 f16), [parity][64 rows] f32 scales.
+struct PgStage {
+  static constexpr int codes = 4096, wscales = 8192, dx = 8448, bytes = 8960, fills = 3;
+};
+
+// ST: stages in flight. The workgroups of an XCD walk K together, so that a step is new
+// to its L2 for all of them. Four stages let four workgroups share a CU; a grid of 512
+// or fewer has at most two per CU and takes eight (1,600 rows: K 2,048 / 3,072, N 1,024,
+// 400 workgroups: 28 / 41.6 us with four, 25 / 36.6 with eight; gate and up, 2,400:
+// 50 and 65). Per layer at 1,600 rows: q|k|v 63 -> 33 us, gate/up 95 -> 50, o 33 -> 25,
+// down 48 -> 37 (before: codes staged through registers, one barrier per step with its
+// loads just ahead, block-diagonal 16 x 16 MFMAs).
+template <int EPI, int ST>
+__global__ void __launch_bounds__(256, ST == 4 ? 4 : 2)
 k_pf_gemm(const uint8_t* __restrict__ w, const uint8_t* __restrict__ w2, int N, int K,
           const int8_t* __restrict__ codes, const float* __restrict__ scales, int S, float* __restrict__ out,
           const float* __restrict__ bias) {
   constexpr bool GLU = EPI == PF_SWIGLU;
-  __shared__ __align__(16) uint8_t s_codes[2][64 * kPfRowBytes];
-  __shared__ float s_dx[2][64 * 2];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int tile = GLU ? blockIdx.x * 2 + (wave & 1) : blockIdx.x * 4 + wave;
-  const uint8_t* mat = (GLU && wave >= 2) ? w2 : w;
-  const int s0 = blockIdx.y * 64;
-  const int bps = K / kPairK;
-  const int j = lane & 15, g = lane >> 4, par = j >> 3;
-  const bool holds = (g >> 1) == par;
-  const int srow = par * 16 + 4 * (lane >> 4);
-  const v4i zero = {0, 0, 0, 0};
-  // staging: thread t loads 16 bytes of row t / 4 (part t % 4); threads < 128 a scale
-  const int st_row = tid >> 2, st_part = tid & 3;
-  const bool st_in = s0 + st_row < S;
-  const int sc_row = tid >> 1, sc_par = tid & 1;
-  const bool sc_in = tid < 128 && s0 + sc_row < S;
-  auto fetch = [&](int bp, v4i& c, float& d) {
-    c = st_in ? *(const v4i*)(codes + (size_t)(s0 + st_row) * K + 64 * bp + 16 * st_part) : zero;
-    d = sc_in ? scales[(size_t)(s0 + sc_row) * (K / 32) + 2 * bp + sc_par] : 0.0f;
+  __shared__ __align__(16) uint8_t s_st[ST * PgStage::bytes];
+  const int tid = threadIdx.x, lane = tid & 63, j = lane & 31, h = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int s0 = blockIdx.y * 64, rb = gridDim.y, bps = K / kPairK;
+  const int ws = wave & 1, wn = wave >> 1;  // the wave's 32 rows, its 32 weight rows (GLU: gate or up)
+  // fills: wave w brings weight unit w, part w of the codes, and the weight scales
+  // (waves 0, 1: half each) or the activation scales of parity w - 2
+  auto unit_of = [&](int u) {
+    if constexpr (GLU) return (u < 2 ? w : w2) + (size_t)(2 * blockIdx.x + (u & 1)) * bps * kUnitBytes;
+    return w + (size_t)(4 * blockIdx.x + u) * bps * kUnitBytes;
   };
-  auto stage = [&](int buf, const v4i& c, float d) {
-    *(v4i*)(s_codes[buf] + st_row * kPfRowBytes + 16 * st_part) = c;
-    if (tid < 128) s_dx[buf][sc_row * 2 + sc_par] = d;
+  const uint8_t* wsrc = unit_of(wave) + 16 * lane;
+  const int8_t* xsrc = codes + ((size_t)(s0 / 64) * 256 + 64 * wave + lane) * 16;
+  const bool act_scale = wave >= 2;
+  const uint8_t* dsrc = act_scale ? (const uint8_t*)(scales + (size_t)(wave & 1) * rb * 64 + s0 + lane)
+                                  : unit_of(lane >> 4) + 1024 + 4 * (lane & 15);
+  const size_t xstep = (size_t)rb * 4096, dstep = act_scale ? (size_t)rb * 512 : (size_t)kUnitBytes;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)s_st;
+  const int ddst = act_scale ? PgStage::dx + 256 * (wave & 1) : PgStage::wscales;  // waves 0 and 1 bring the same bytes
+  auto fill = [&](int bp) {  // past the last pair: the last one again, into a stage nobody reads
+    const uint32_t st = lds0 + (bp % ST) * PgStage::bytes;
+    const int at = min(bp, bps - 1);
+    lds_fill16(wsrc + (size_t)at * kUnitBytes, st + wave * 1024);
+    lds_fill16(xsrc + at * xstep, st + PgStage::codes + wave * 1024);
+    lds_fill4(dsrc + at * dstep, st + ddst);
   };
-  v4i nc;
-  float nd;
-  fetch(0, nc, nd);
-  stage(0, nc, nd);
-  float part[8][4], tot[8][4];
+  const int ut = 2 * wn + (j >> 4);  // lane j holds weight row j of 32, in this unit
+  float part[2][16], tot[2][16];     // [parity][register]
 #pragma unroll
-  for (int cg = 0; cg < 8; ++cg)
+  for (int p = 0; p < 2; ++p)
 #pragma unroll
-    for (int q = 0; q < 4; ++q) part[cg][q] = tot[cg][q] = 0.0f;
-  // the weight unit of the next pair is in flight while a pair computes
-  const uint8_t* wtile = mat + (size_t)tile * bps * kUnitBytes;
-  v4i na = __builtin_nontemporal_load((const v4i*)(wtile + lane * 16));
-  uint2 nsw = *(const uint2*)(wtile + 1024 + srow * 2);
-  int sl = 0, sl_end = bps / 4;
-  for (int bp = 0; bp < bps; ++bp) {
-    const int buf = bp & 1;
-    if (bp + 1 < bps) fetch(bp + 1, nc, nd);
-    const v4i a = na;
-    const uint2 sw = nsw;
-    if (bp + 1 < bps) {
-      const uint8_t* unit = wtile + (size_t)(bp + 1) * kUnitBytes;
-      na = __builtin_nontemporal_load((const v4i*)(unit + lane * 16));
-      nsw = *(const uint2*)(unit + 1024 + srow * 2);
-    }
-    float dw[4];
-    dw[0] = half_bits_to_float((uint16_t)(sw.x & 0xffff));
-    dw[1] = half_bits_to_float((uint16_t)(sw.x >> 16));
-    dw[2] = half_bits_to_float((uint16_t)(sw.y & 0xffff));
-    dw[3] = half_bits_to_float((uint16_t)(sw.y >> 16));
-    __syncthreads();  // the staged pair bp is complete
+    for (int r = 0; r < 16; ++r) part[p][r] = tot[p][r] = 0.0f;
+  const v16i zero = {};
 #pragma unroll
-    for (int cg = 0; cg < 8; ++cg) {
-      const int row = 8 * cg + (j & 7);
-      const v4i b = holds ? *(const v4i*)(s_codes[buf] + row * kPfRowBytes + 32 * par + 16 * (g & 1)) : zero;
-      const float dx = s_dx[buf][row * 2 + par];
-      const v4i c = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b, zero, 0, 0, 0);
+  for (int i = 0; i < ST - 1; ++i) fill(i);
+#pragma unroll 1
+  for (int sl = 0, bp = 0; sl < 4; ++sl) {
+#pragma unroll 1
+    for (const int end = bps * (sl + 1) / 4; bp < end; ++bp) {
+      // this wave's fills of pair bp are done (those of later pairs may be in flight);
+      // behind the barrier everyone's are, and nobody reads pair bp - 1 any more
+      asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((ST - 2) * PgStage::fills) : "memory");
+      fill(bp + ST - 1);
+      const uint8_t* st = s_st + (bp % ST) * PgStage::bytes;
 #pragma unroll
-      for (int q = 0; q < 4; ++q) part[cg][q] = fmaf((float)c[q], dw[q] * dx, part[cg][q]);
-    }
-    if (bp + 1 == sl_end) {  // a K-slice ends: fold it into the running total
+      for (int p = 0; p < 2; ++p) {
+        const v4i a = *(const v4i*)(st + PgStage::codes + (2 * p + h) * 1024 + 16 * (32 * ws + j));
+        const v4i bw = *(const v4i*)(st + ut * 1024 + (2 * p + h) * 256 + 16 * (j & 15));
+        const float dw = half_bits_to_float(*(const uint16_t*)(st + PgStage::wscales + ut * 64 + 2 * (16 * p + (j & 15))));
+        const v16i c = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, bw, zero, 0, 0, 0);
 #pragma unroll
-      for (int cg = 0; cg < 8; ++cg)
+        for (int i = 0; i < 4; ++i) {  // registers 4 i + e: rows 8 i + 4 h + e
+          const v4f dx = *(const v4f*)(st + PgStage::dx + 4 * (64 * p + 32 * ws + 8 * i + 4 * h));
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          tot[cg][q] = sl == 0 ? part[cg][q] : __fadd_rn(tot[cg][q], part[cg][q]);
-          part[cg][q] = 0.0f;
+          for (int e = 0; e < 4; ++e) part[p][4 * i + e] = fmaf((float)c[4 * i + e], dw * dx[e], part[p][4 * i + e]);
         }
-      ++sl;
-      sl_end = (bps * (sl + 1)) / 4;
+      }
     }
-    if (bp + 1 < bps) stage(buf ^ 1, nc, nd);  // the other buffer: read two steps ago, behind the barrier
+    // a K-slice ends: fold it into the running total (0 + s0 is s0: no sum is -0)
+#pragma unroll
+    for (int p = 0; p < 2; ++p)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        tot[p][r] = __fadd_rn(tot[p][r], part[p][r]);
+        part[p][r] = 0.0f;
+      }
   }
+  float y[16];
 #pragma unroll
-  for (int cg = 0; cg < 8; ++cg)
-#pragma unroll
-    for (int q = 0; q < 4; ++q) tot[cg][q] = __fadd_rn(tot[cg][q], dpp_f<kDppRor8>(tot[cg][q]));  // even + odd
+  for (int r = 0; r < 16; ++r) y[r] = __fadd_rn(tot[0][r], tot[1][r]);  // even + odd
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no fill outlives the workgroup
   if constexpr (GLU) {
-    // the up waves hand their values to the gate waves of the same tile
+    // the up waves hand their values to the gate waves of the same rows
     __syncthreads();
-    __shared__ __align__(16) float s_up[2 * 8 * 64 * 4];  // [2 tiles][8 cg][64 lanes][4]
-    if (wave >= 2)
+    v4f* s_up = (v4f*)s_st + (ws * 64 + lane) * 4;
+    if (wn == 1) {
 #pragma unroll
-      for (int cg = 0; cg < 8; ++cg)
-        *(v4f*)(s_up + (((wave & 1) * 8 + cg) * 64 + lane) * 4) = (v4f){tot[cg][0], tot[cg][1], tot[cg][2], tot[cg][3]};
-    __syncthreads();
-    if (wave >= 2) return;
-#pragma unroll
-    for (int cg = 0; cg < 8; ++cg) {
-      const v4f u = *(const v4f*)(s_up + (((wave & 1) * 8 + cg) * 64 + lane) * 4);
-#pragma unroll
-      for (int q = 0; q < 4; ++q) tot[cg][q] = dev_swiglu(tot[cg][q], u[q]);
+      for (int i = 0; i < 4; ++i) s_up[i] = v4f{y[4 * i], y[4 * i + 1], y[4 * i + 2], y[4 * i + 3]};
     }
+    __syncthreads();
+    if (wn == 1) return;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) y[r] = dev_swiglu(y[r], s_up[r / 4][r % 4]);
   }
-  // lanes j and j + 8 hold the same sums: lane j takes row groups 0..3 of
-  // rows s0 + 8 cg + j, lane j + 8 groups 4..7
-  {
-    const int n = tile * 16 + 4 * (lane >> 4), hi = j >> 3;
-    // a mask the compiler cannot see through: a plain select between tot[c] and
-    // tot[4 + c] becomes a lane-dependent index into tot, which moves tot to
-    // scratch memory for the whole kernel
-    uint32_t m = 0u - (uint32_t)hi;
-    asm volatile("" : "+v"(m));
-    float y[4][4];
+  const int n = GLU ? 32 * (int)blockIdx.x + j : 64 * (int)blockIdx.x + 32 * wn + j;
+  if constexpr (EPI >= PF_BIAS) {
+    // linear = mul_mat + bias, then the activation or the residual add
+    const float bn = bias[n];
 #pragma unroll
-    for (int c = 0; c < 4; ++c)
+    for (int r = 0; r < 16; ++r) y[r] = __fadd_rn(y[r], bn);
+    if constexpr (EPI == PF_BIAS_GELU) {
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const uint32_t lo = __float_as_uint(tot[c][q]);
-        y[c][q] = __uint_as_float(lo ^ ((lo ^ __float_as_uint(tot[4 + c][q])) & m));
+      for (int r = 0; r < 16; r += 8) {
+        float e[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) e[i] = y[r + i];
+        dev_gelu_erf_n<8>(e);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) y[r + i] = e[i];
       }
-    if constexpr (EPI >= PF_BIAS) {
-      // linear = mul_mat + bias, then the activation or the residual add
-      const v4f b = *(const v4f*)(bias + n);
-#pragma unroll
-      for (int c = 0; c < 4; ++c)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) y[c][q] = __fadd_rn(y[c][q], b[q]);
-      if constexpr (EPI == PF_BIAS_GELU) {
-#pragma unroll
-        for (int c = 0; c < 4; c += 2) {
-          float g[8];
-#pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            g[q] = y[c][q];
-            g[4 + q] = y[c + 1][q];
-          }
-          dev_gelu_erf_n<8>(g);
-#pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            y[c][q] = g[q];
-            y[c + 1][q] = g[4 + q];
-          }
-        }
-      }
-      if constexpr (EPI == PF_BIAS_SILU)
-#pragma unroll
-        for (int c = 0; c < 4; ++c)
-#pragma unroll
-          for (int q = 0; q < 4; ++q) y[c][q] = dev_silu(y[c][q]);
     }
+    if constexpr (EPI == PF_BIAS_SILU)
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      const int row = s0 + 8 * (4 * hi + c) + (j & 7);
-      if (row >= S) continue;
-      float* dst = out + (size_t)row * N + n;
-      v4f v;
-      if constexpr (EPI == PF_RESID || EPI == PF_BIAS_RESID) {
-        const v4f x = *(const v4f*)dst;
+      for (int r = 0; r < 16; ++r) y[r] = dev_silu(y[r]);
+  }
 #pragma unroll
-        for (int q = 0; q < 4; ++q) v[q] = __fadd_rn(x[q], y[c][q]);
-      } else {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) v[q] = y[c][q];
-      }
-      *(v4f*)dst = v;
-    }
+  for (int r = 0; r < 16; ++r) {
+    const int row = s0 + 32 * ws + 8 * (r / 4) + 4 * h + r % 4;
+    if (row >= S) continue;
+    float* dst = out + (size_t)row * N + n;
+    *dst = (EPI == PF_RESID || EPI == PF_BIAS_RESID) ? __fadd_rn(*dst, y[r]) : y[r];
   }
 }
 
@@ -372,8 +344,12 @@ void launch_pf_quant(hipStream_t s, const float* src, int S, int K, int8_t* code
 void launch_pf_gemm(hipStream_t s, int epi, const uint8_t* w, const uint8_t* w2, int N, int K, const int8_t* codes,
                     const float* scales, int S, float* out, const float* bias) {
   const dim3 blocks((unsigned)(epi == PF_SWIGLU ? N / 32 : N / 64), (unsigned)((S + 63) / 64));
-#define MTG_PF_GEMM(E) \
-  hipLaunchKernelGGL(k_pf_gemm<E>, blocks, dim3(256), 0, s, w, w2, N, K, codes, scales, S, out, bias)
+  const bool deep = (size_t)blocks.x * blocks.y <= 512;  // two workgroups per CU or fewer
+#define MTG_PF_GEMM(E)                                                                                         \
+  if (deep)                                                                                                    \
+    hipLaunchKernelGGL((k_pf_gemm<E, 8>), blocks, dim3(256), 0, s, w, w2, N, K, codes, scales, S, out, bias);  \
+  else                                                                                                         \
+    hipLaunchKernelGGL((k_pf_gemm<E, 4>), blocks, dim3(256), 0, s, w, w2, N, K, codes, scales, S, out, bias)
   switch (epi) {
     case PF_STORE: MTG_PF_GEMM(PF_STORE); break;
     case PF_RESID: MTG_PF_GEMM(PF_RESID); break;
