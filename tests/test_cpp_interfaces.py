@@ -33,3 +33,8 @@ def test_cpp_speculative_gate_on_gpu():
     print("C++ speculative gate: 2-layer q8_0 model, 40 tokens, forced rejections", flush=True)
     rec = _run("test_speculative_gate", 100)
     assert rec["passed"] and rec["tokens"] == 40
+
+
+def test_erf_polynomials_round_as_the_series():
+    rec = _run("test_erf_poly", 100)
+    assert rec["differ"] == 0 and rec["floats"] > 17_000_000
