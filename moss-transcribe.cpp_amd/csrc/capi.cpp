@@ -618,6 +618,8 @@ void mtg_q8_free(mtg_q8_packed* p) {
 
 int mtg_q8_mul_mat_dev(const mtg_q8_packed* w, const float* x_dev, int32_t T, float* y_dev) {
   if (!w || !x_dev || !y_dev || T <= 0 || T > MTG_MAX_BATCH) return MTG_ERR_INVALID;
+  if (mtg::launch_mul_mat(nullptr, w->tiles, w->n, w->k, x_dev, T, y_dev))
+    return hipDeviceSynchronize() == hipSuccess ? MTG_OK : MTG_ERR_DEVICE;
   mtg::StepDesc host{};
   host.T = T;
   host.groups = (T + 7) / 8;

@@ -167,6 +167,114 @@ k_gemm(const StepDesc* __restrict__ desc, const uint8_t* __restrict__ w,
   }
 }
 
+// ------------------------------------------------------ one product alone ---
+// y[t][row] for T <= 16 activation rows, from f32 rows to f32 rows in one launch without
+// scratch memory: every workgroup converts the rows to q8_0 in LDS (codes of the 8 rows
+// of a column group: 512 bytes per block pair, row t's 16-byte part p of 4 at p * 128 +
+// (t % 8) * 16) and then works off 16-row weight tiles. SPLIT: the four waves take the
+// four K-slices of the workgroup's tile and meet in LDS; else a wave takes whole tiles.
+// What bounds it: for 1024 x 1024 and one row the call (a launch and the wait for it);
+// its three allocations, two copies, two launches and three frees took 33 us, this 14.
+// For many tiles, the weights from memory.
+constexpr int kMulMatLds = 128 * 1024;  // panel limit: K up to 14,528 (8 rows) or 7,232 (16 rows)
+constexpr size_t mul_mat_panel_bytes(int bps, int G) { return (size_t)bps * G * (512 + 64); }
+
+template <int G, bool SPLIT>
+__global__ void __launch_bounds__(256)
+k_mul_mat(const uint8_t* __restrict__ w, int n, int bps, const float* __restrict__ x, int T, float* __restrict__ y) {
+  extern __shared__ v4i mm_lds_v4[];
+  __shared__ float red[SPLIT ? 4 : 1][SPLIT ? G * 4 : 1][64];
+  uint8_t* s_codes = (uint8_t*)mm_lds_v4;                     // [bps][G][512]
+  float* s_scales = (float*)(s_codes + (size_t)bps * G * 512);  // [bps][G][parity * 8 + row]
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int K = bps * kPairK, quads = K / 4;
+  // 8 lanes convert a block, 4 elements each, four rows' loads in flight
+  for (int qd = tid; qd < quads; qd += 256) {
+    const int k = 4 * qd;
+    for (int t0 = 0; t0 < T; t0 += 4) {
+      v4f v4[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v4[i] = *(const v4f*)(x + (size_t)min(t0 + i, T - 1) * K + k);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int t = t0 + i, at = (k >> 6) * G + (t >> 3);
+        if (t >= T) break;
+        const float v[4] = {v4[i][0], v4[i][1], v4[i][2], v4[i][3]};
+        int8_t q[4];
+        const float d = quant_block8(v, q);
+        *(uint32_t*)(s_codes + (size_t)at * 512 + ((k >> 4) & 3) * 128 + (t & 7) * 16 + (k & 15)) =
+            (uint32_t)(uint8_t)q[0] | ((uint32_t)(uint8_t)q[1] << 8) | ((uint32_t)(uint8_t)q[2] << 16) |
+            ((uint32_t)(uint8_t)q[3] << 24);
+        if ((qd & 7) == 0) s_scales[at * 16 + ((k >> 5) & 1) * 8 + (t & 7)] = d;
+      }
+    }
+  }
+  __syncthreads();
+  const int j = lane & 15, g = lane >> 4, par = j >> 3;
+  const bool holds = (g >> 1) == par;  // the block-diagonal B operand: zeros elsewhere
+  const v4i zero = {0, 0, 0, 0};
+  auto slice = [&](const uint8_t* tile, int sl, float (&acc)[G][4]) {
+#pragma unroll
+    for (int cg = 0; cg < G; ++cg)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[cg][r] = 0.0f;
+#pragma unroll 4
+    for (int bp = bps * sl / 4; bp < bps * (sl + 1) / 4; ++bp) {
+      const uint8_t* unit = tile + (size_t)bp * kUnitBytes;
+      const v4i a = *(const v4i*)(unit + lane * 16);
+      const uint2 sw = *(const uint2*)(unit + 1024 + (par * 16 + 4 * g) * 2);
+      const float dw[4] = {half_bits_to_float((uint16_t)(sw.x & 0xffff)), half_bits_to_float((uint16_t)(sw.x >> 16)),
+                           half_bits_to_float((uint16_t)(sw.y & 0xffff)), half_bits_to_float((uint16_t)(sw.y >> 16))};
+#pragma unroll
+      for (int cg = 0; cg < G; ++cg) {
+        const int at = bp * G + cg;
+        const v4i b = holds ? *(const v4i*)(s_codes + (size_t)at * 512 + g * 128 + (j & 7) * 16) : zero;
+        const float dx = s_scales[at * 16 + j];
+        const v4i c = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b, zero, 0, 0, 0);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[cg][r] = fmaf((float)c[r], dw[r] * dx, acc[cg][r]);
+      }
+    }
+  };
+  auto store = [&](int tile, float (&acc)[G][4]) {
+#pragma unroll
+    for (int cg = 0; cg < G; ++cg) {
+      v4f o;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o[r] = __fadd_rn(acc[cg][r], dpp_f<kDppRor8>(acc[cg][r]));  // even + odd
+      const int t = cg * 8 + j;
+      if (j < 8 && t < T) *(v4f*)(y + (size_t)t * n + tile * 16 + 4 * g) = o;
+    }
+  };
+  if constexpr (SPLIT) {
+    const int tile = blockIdx.x;
+    float acc[G][4];
+    slice(w + (size_t)tile * bps * kUnitBytes, wave, acc);
+#pragma unroll
+    for (int i = 0; i < G * 4; ++i) red[wave][i][lane] = acc[i / 4][i % 4];
+    __syncthreads();
+    if (wave) return;
+#pragma unroll
+    for (int i = 0; i < G * 4; ++i)
+      acc[i / 4][i % 4] = __fadd_rn(__fadd_rn(__fadd_rn(acc[i / 4][i % 4], red[1][i][lane]), red[2][i][lane]), red[3][i][lane]);
+    store(tile, acc);
+  } else {
+    for (int tile = blockIdx.x * 4 + wave; tile < n / 16; tile += 4 * gridDim.x) {
+      const uint8_t* wt = w + (size_t)tile * bps * kUnitBytes;
+      float acc[G][4], part[G][4];
+      slice(wt, 0, acc);
+      for (int sl = 1; sl < 4; ++sl) {
+        slice(wt, sl, part);
+#pragma unroll
+        for (int cg = 0; cg < G; ++cg)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) acc[cg][r] = __fadd_rn(acc[cg][r], part[cg][r]);
+      }
+      store(tile, acc);
+    }
+  }
+}
+
 // ------------------------------------------------- q/k norm, rope, append ---
 // grid (16 rows, n_heads + 2*n_kv_heads units), one wave per unit; lane i owns
 // the NEOX pair (i, i + 64) of head_dim 128.
@@ -836,6 +944,35 @@ static void gemm_launch(hipStream_t s, int G, const StepDesc* desc, const uint8_
   else
     hipLaunchKernelGGL((k_gemm<EPI, SPLIT, 2>), dim3(tiles), dim3(SPLIT * 64), 0, s, desc, w, w2, n,
                        bps, x, out);
+}
+
+bool launch_mul_mat(hipStream_t s, const uint8_t* w, int n, int k, const float* x, int T, float* y) {
+  const int bps = k / kPairK, G = (T + 7) / 8, tiles = n / 16;
+  const size_t lds = mul_mat_panel_bytes(bps, G);
+  if (lds > (size_t)kMulMatLds || ((uintptr_t)x | (uintptr_t)y) % 16) return false;
+  // A workgroup per tile while converting the panel that often is cheap; else 1,024
+  // workgroups walk the tiles, which streams as fast as the general path only with four
+  // panels to a CU (K 4,096, 16 rows, N 16,384: 56 us against the general path's 47; 8
+  // rows: 37 against 46; K 1,024, N 151,936, one row: 38 against 55).
+  const bool split = tiles <= 1024 && (int64_t)tiles * T * k <= (1 << 25);
+  if (4 * lds > 150 * 1024 && tiles > 512) return false;
+  const dim3 grid((unsigned)(split ? tiles : std::min((tiles + 3) / 4, 1024)));
+#define MTG_MUL_MAT(G_, SPLIT_)                                                                                       \
+  do {                                                                                                                \
+    if (lds + 8192 > 65536 && hipFuncSetAttribute((const void*)k_mul_mat<G_, SPLIT_>,                                 \
+                                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) \
+      return false;                                                                                                   \
+    hipLaunchKernelGGL((k_mul_mat<G_, SPLIT_>), grid, dim3(256), lds, s, w, n, bps, x, T, y);                         \
+  } while (0)
+  if (G == 1) {
+    if (split) MTG_MUL_MAT(1, true);
+    else MTG_MUL_MAT(1, false);
+  } else {
+    if (split) MTG_MUL_MAT(2, true);
+    else MTG_MUL_MAT(2, false);
+  }
+#undef MTG_MUL_MAT
+  return true;
 }
 
 void launch_gemm_store(hipStream_t s, int G, const StepDesc* desc, const uint8_t* w, int n, int k,
