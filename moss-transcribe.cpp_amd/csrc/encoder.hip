@@ -375,6 +375,7 @@ int mtg_encoder_create(const mtg_encoder_desc* d, mtg_encoder** out) {
   int rc = e->check(hipStreamCreateWithFlags(&e->stream, hipStreamNonBlocking), "stream");
   if (!rc) rc = e->check(hipEventCreate(&e->ev0), "event");
   if (!rc) rc = e->check(hipEventCreate(&e->ev1), "event");
+  if (!rc) rc = e->check(prepare_kernels_pf_wt(), "kernel attributes");
   // staging for the raw q8_0 rows of the largest matrix
   size_t raw_max = (size_t)std::max(F, std::max(D, H)) * (std::max(F, IN) / 32) * 34;
   uint8_t* staging = rc ? nullptr : (uint8_t*)e->dalloc(raw_max);

@@ -124,6 +124,7 @@ void launch_pf_gemm_wt(hipStream_t s, int wtype, int epi, const uint8_t* w, cons
                        const WtAct& act, int S, float* out, const float* bias = nullptr);
 // the K this GEMM takes: f16 and f32 1,024 / 2,048 / 3,072 / 4,096; q4_K any multiple of 256
 int pf_gemm_wt_supported(int wtype, int K);
+hipError_t prepare_kernels_pf_wt();
 
 // ---- f16 / q4_K weights (kernels_wt.hip); weights in the GGUF row layout ----
 bool wt_shape_supported(int wtype, int k);

@@ -4,7 +4,7 @@
 // as prefill.hip does for q8_0. Per layer:
 //   k_pf_act_wt     RMSNorm * gain (or the rows as they are) and the weight type's
 //                   vec_dot_type: f16 values, or q8_K blocks (quantize_row_q8_K)
-//   k_pf_gemm_f16   f16 weights x f16 activations on f32 MFMA, in the canonical
+//   k_pf_gemm_f16   f16 (f32) weights x f16 (f32) activations on f32 MFMA, in the canonical
 //                   segment order (below)
 //   k_pf_gemm_q4k   q4_K weights x q8_K activations: exact int32 sums per
 //                   superblock on int8 MFMA, the float chain over superblocks
@@ -86,161 +86,197 @@ __device__ __forceinline__ void pf_store4(int epi, float* out, int N, int t, int
 }
 
 // ------------------------------------------------------- f16 / f32 GEMM ----
-// out[s][n] for 64 weight rows x 64 activation rows per workgroup (wave w: the
-// 16-row tile 4 blockIdx.x + w; for the SwiGLU epilogue waves 0, 1 take gate rows
-// 32 blockIdx.x + 16 w and waves 2, 3 the same rows of up, meeting in LDS).
-// The canonical f16 dot (the oracle's mul_mat_f16, the per-op k_gemm_f16): K in
-// 64 consecutive segments of L = K / 64 elements, each an fma chain from 0 over
-// its elements in order (a product of two f16 values is exact in f32), the 64
-// partials reduced by the xor butterfly (v[i] + v[i ^ 32], then 16, .. 1, lane 0).
+// out[s][n] in the canonical f16 dot (the oracle's mul_mat_f16, the per-op k_gemm_f16):
+// K in 64 consecutive segments of L = K / 64 elements, each an fma chain from 0 over
+// its elements in order (a product of two f16 values is exact in f32), the 64 partials
+// reduced by the xor butterfly (v[i] + v[i ^ 32], then 16, .. 1, lane 0).
 // v_mfma_f32_16x16x4f32 returns fma(a3, b3, fma(a2, b2, fma(a1, b1, fma(a0, b0, c))))
-// per output, so L / 4 chained MFMAs from a zero accumulator are one segment's
-// chain (k-step s: elements 4 s + kk held by lane group kk). The segments run in
-// 6-bit bit-reversed order: the butterfly's tree is then the balanced binary tree
-// over the run, folded as it goes with a stack of six partials (a binary counter).
-// Every segment's weight and activation rows are staged in LDS as f32 (row stride
-// L + 4 floats: the operand reads of a wave hit 64 distinct banks), the next
-// segment's rows already in flight in registers.
-// F32: f32 weights and activations (vec_dot_type F32), the same segments, MFMA
-// chains and tree: each step of a segment's chain is one fma of two f32 values,
-// as the oracle's mul_mat_f32 and the per-op k_gemm_f32 take it.
+// per output, so L / 4 chained MFMAs from a zero accumulator are one segment's chain
+// (k-step s: elements 4 s + kk held by lane group kk). The segments run in 6-bit
+// bit-reversed order: the butterfly's tree is then the balanced binary tree over the
+// run, folded as it goes with a stack of partials (a binary counter).
+// F32: f32 weights and activations (vec_dot_type F32), the same segments, chains and
+// tree: each step of a segment's chain is one fma of two f32 values, as the oracle's
+// mul_mat_f32 and the per-op k_gemm_f32 take it.
+//
+// What bounds it: f32 MFMAs (33 cycles each) and every vector instruction beside them,
+// which do not overlap: 420 us per decoder layer of 2,048 rows for the MFMAs alone. So a
+// wave takes 32 weight rows x 32 activation rows (four chains; one 16-byte LDS read
+// feeds four k-steps of two of them), 64 elements of the rows are staged per barrier,
+// converted once per workgroup, the next 64 in flight in registers, and the first tree
+// levels, those inside a stage, are plain sums. NW waves: 16 NW weight rows x 64
+// activation rows; 8 where that leaves every CU a workgroup (its loads per MFMA are
+// three quarters of 4's), else 4.
+// Per layer of 2,048 rows, f16: q|k|v 237 -> 173 us, gate/up 345 -> 261, o 114 -> 85, down
+// 165 -> 130 (before: 16 x 64 tiles per wave, one 4-byte LDS read per operand and MFMA, a
+// barrier and a six-level fold per segment).
 __device__ __forceinline__ int bitrev6(int k) { return (int)(__builtin_bitreverse32((uint32_t)k) >> 26); }
 
-template <bool GLU, int L, bool F32 = false>
-__global__ void __launch_bounds__(256)
+template <int L, int NW>
+struct PfF16 {
+  static constexpr int LPS = L == 16 ? 4 : L == 32 ? 2 : 1;  // segments per stage
+  static constexpr int LV = LPS == 4 ? 2 : LPS == 2 ? 1 : 0;  // their tree levels
+  static constexpr int rows = 16 * NW + 64, stride = L + 4;    // staged rows; floats per row (bank spread)
+  static constexpr int leaf = rows * stride, stage = LPS * leaf;
+  static constexpr size_t bytes = (size_t)2 * stage * 4;
+};
+
+template <bool GLU, int L, bool F32, int NW>
+__global__ void __launch_bounds__(64 * NW, 2)
 k_pf_gemm_f16(const void* __restrict__ wv, const void* __restrict__ w2v, int N, const void* __restrict__ xv, int S,
               float* __restrict__ out, int epi, const float* __restrict__ bias) {
+  using P = PfF16<L, NW>;
   using E = typename std::conditional<F32, float, uint16_t>::type;
   constexpr int EP = 16 / (int)sizeof(E);  // elements per 16-byte piece
-  constexpr int K = 64 * L, LS = L + 4, NP = L / EP;  // pieces per row and segment
-  constexpr int NPIECE = 2 * 64 * NP, PPT = (NPIECE + 255) / 256;
+  constexpr int K = 64 * L, NP = L / EP, WR = 16 * NW, GR = WR / 2;  // pieces per row and segment; weight rows; gate rows
+  constexpr int NPIECE = P::LPS * P::rows * NP, PPT = (NPIECE + 64 * NW - 1) / (64 * NW);
+  extern __shared__ v4f pf16_lds_v4[];
+  float* const s_st = (float*)pf16_lds_v4;
   const E* w = (const E*)wv;
   const E* w2 = (const E*)w2v;
   const E* x = (const E*)xv;
-  __shared__ __align__(16) float s_w[2][64 * LS];
-  __shared__ __align__(16) float s_x[2][64 * LS];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, m = lane & 15, kk = lane >> 4;
+  const int tid = threadIdx.x, lane = tid & 63, m = lane & 15, kk = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wn = wave >> 1, ws = wave & 1;
   const int s0 = blockIdx.y * 64;
-  // weight row r (< 64) of the workgroup
-  auto wrow = [&](int r) -> const E* {
-    if constexpr (GLU) return (r < 32 ? w : w2) + (size_t)(32 * blockIdx.x + (r & 31)) * K;
-    return w + (size_t)(64 * blockIdx.x + r) * K;
+  // staged row r: weight rows first (GLU: gate, then up), then the activation's 64;
+  // rows past the matrix or the block read the last one, their outputs are dropped
+  const int nrow = GLU ? GR * (int)blockIdx.x : WR * (int)blockIdx.x;
+  auto row_of = [&](int r) -> const E* {
+    if (r >= WR) return x + (size_t)min(s0 + r - WR, S - 1) * K;
+    if constexpr (GLU) return (r < GR ? w : w2) + (size_t)min(nrow + r % GR, N - 1) * K;
+    return w + (size_t)min(nrow + r, N - 1) * K;
   };
-  uint4 reg[PPT];
-  auto fetch = [&](int seg) {
+  const E* src[PPT];
+  int dst[PPT], leaf[PPT];
 #pragma unroll
-    for (int i = 0; i < PPT; ++i) {
-      const int p = tid + 256 * i;
-      if (p < NPIECE) {
-        const int half = p / (64 * NP), q = p % (64 * NP), r = q / NP, j = q % NP;
-        if (half == 0)
-          reg[i] = *(const uint4*)(wrow(r) + seg * L + EP * j);
-        else
-          reg[i] = s0 + r < S ? *(const uint4*)(x + (size_t)(s0 + r) * K + seg * L + EP * j) : make_uint4(0, 0, 0, 0);
-      }
-    }
-  };
-  auto stage = [&](int buf) {
-#pragma unroll
-    for (int i = 0; i < PPT; ++i) {
-      const int p = tid + 256 * i;
-      if (p < NPIECE) {
-        const int half = p / (64 * NP), q = p % (64 * NP), r = q / NP, j = q % NP;
-        float* dst = (half ? s_x[buf] : s_w[buf]) + r * LS + EP * j;
-        const uint32_t u[4] = {reg[i].x, reg[i].y, reg[i].z, reg[i].w};
-        if constexpr (F32) {
-          *(v4f*)dst = v4f{__uint_as_float(u[0]), __uint_as_float(u[1]), __uint_as_float(u[2]), __uint_as_float(u[3])};
-          continue;
-        }
-        v4f lo, hi;
-#pragma unroll
-        for (int e = 0; e < 2; ++e) {
-          lo[2 * e] = half_bits_to_float((uint16_t)(u[e] & 0xffffu));
-          lo[2 * e + 1] = half_bits_to_float((uint16_t)(u[e] >> 16));
-          hi[2 * e] = half_bits_to_float((uint16_t)(u[2 + e] & 0xffffu));
-          hi[2 * e + 1] = half_bits_to_float((uint16_t)(u[2 + e] >> 16));
-        }
-        *(v4f*)dst = lo;
-        *(v4f*)(dst + 4) = hi;
-      }
-    }
-  };
-  v4f stk[6][4], res[4];
-#pragma unroll
-  for (int ct = 0; ct < 4; ++ct) {
-    res[ct] = v4f{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int lvl = 0; lvl < 6; ++lvl) stk[lvl][ct] = res[ct];
+  for (int i = 0; i < PPT; ++i) {
+    const int p = min(tid + 64 * NW * i, NPIECE - 1), q = p / NP, j = p % NP, r = q % P::rows;
+    leaf[i] = q / P::rows;
+    src[i] = row_of(r) + EP * j;
+    dst[i] = leaf[i] * P::leaf + r * P::stride + (EP / 4) * j;  // element 4 s + e of the segment at e * L / 4 + s
   }
-  fetch(bitrev6(0));
-  stage(0);
-  for (int k = 0; k < 64; ++k) {
-    const int buf = k & 1;
-    if (k + 1 < 64) fetch(bitrev6(k + 1));
-    __syncthreads();  // segment k is staged; the other buffer's readers (segment k - 1) are done
-    const float* aw = s_w[buf] + (16 * wave + m) * LS + kk;
-    v4f cur[4];
+  uint4 reg[PPT];
+  auto fetch = [&](int st) {
 #pragma unroll
-    for (int ct = 0; ct < 4; ++ct) cur[ct] = v4f{0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < PPT; ++i) reg[i] = *(const uint4*)(src[i] + bitrev6(P::LPS * st + leaf[i]) * L);
+  };
+  auto stage = [&](float* buf) {
 #pragma unroll
-    for (int s = 0; s < L / 4; ++s) {
-      const float av = aw[4 * s];
+    for (int i = 0; i < PPT; ++i) {
+      if (NPIECE % (64 * NW) && tid + 64 * NW * i >= NPIECE) continue;
+      float* d = buf + dst[i];
+      const uint32_t u[4] = {reg[i].x, reg[i].y, reg[i].z, reg[i].w};
+      if constexpr (F32) {
 #pragma unroll
-      for (int ct = 0; ct < 4; ++ct)
-        cur[ct] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, s_x[buf][(16 * ct + m) * LS + 4 * s + kk], cur[ct], 0, 0, 0);
+        for (int e = 0; e < 4; ++e) d[e * (L / 4)] = __uint_as_float(u[e]);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int sh = 16 * (e & 1);
+          *(float2*)(d + e * (L / 4)) = make_float2(half_bits_to_float((uint16_t)(u[e / 2] >> sh)),
+                                                    half_bits_to_float((uint16_t)(u[2 + e / 2] >> sh)));
+        }
+      }
     }
-    // fold leaf k into the stack: while bit lvl of k is set, the left sibling
-    // (the earlier subtree) is added; the first clear bit keeps the partial
+  };
+  v4f stk[6 - P::LV][4];  // tile 2 a + b: weight rows 16 a, activation rows 16 b of the wave's 32 x 32
+  v4f res[4];
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    res[c] = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int lvl = 0; lvl < 6 - P::LV; ++lvl) stk[lvl][c] = res[c];
+  }
+  auto add = [](v4f (&a)[4], const v4f (&b)[4]) {  // a = b + a, per output
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) a[c][q] = __fadd_rn(b[c][q], a[c][q]);
+  };
+  const int aoff = (32 * wn + m) * P::stride + kk * (L / 4), boff = (WR + 32 * ws + m) * P::stride + kk * (L / 4);
+  auto segment = [&](const float* lf, v4f (&cur)[4]) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c) cur[c] = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int q = 0; q < L / 16; ++q) {
+      v4f a[2], b[2];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        a[h] = *(const v4f*)(lf + aoff + 16 * h * P::stride + 4 * q);
+        b[h] = *(const v4f*)(lf + boff + 16 * h * P::stride + 4 * q);
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+          cur[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[c >> 1][e], b[c & 1][e], cur[c], 0, 0, 0);
+    }
+  };
+  fetch(0);
+  stage(s_st);
+  constexpr int NST = 64 / P::LPS;
+  for (int st = 0; st < NST; ++st) {
+    const float* buf = s_st + (st & 1) * P::stage;
+    if (st + 1 < NST) fetch(st + 1);
+    __syncthreads();  // stage st is complete; the other buffer's readers (stage st - 1) are done
+    v4f cur[4];
+    segment(buf, cur);
+    if constexpr (P::LPS >= 2) {
+      v4f nxt[4];
+      segment(buf + P::leaf, nxt);
+      add(cur, nxt);
+    }
+    if constexpr (P::LPS == 4) {
+      v4f c2[4], c3[4];
+      segment(buf + 2 * P::leaf, c2);
+      segment(buf + 3 * P::leaf, c3);
+      add(c2, c3);
+      add(cur, c2);
+    }
+    // fold: while bit lvl of st is set, the left sibling (the earlier subtree) is added;
+    // the first clear bit keeps the partial
     bool carry = true;
 #pragma unroll
-    for (int lvl = 0; lvl < 6; ++lvl) {
+    for (int lvl = 0; lvl < 6 - P::LV; ++lvl) {
       if (carry) {
-        if ((k >> lvl) & 1) {
-#pragma unroll
-          for (int ct = 0; ct < 4; ++ct)
-#pragma unroll
-            for (int q = 0; q < 4; ++q) cur[ct][q] = __fadd_rn(stk[lvl][ct][q], cur[ct][q]);
+        if ((st >> lvl) & 1) {
+          add(cur, stk[lvl]);
         } else {
 #pragma unroll
-          for (int ct = 0; ct < 4; ++ct) stk[lvl][ct] = cur[ct];
+          for (int c = 0; c < 4; ++c) stk[lvl][c] = cur[c];
           carry = false;
         }
       }
     }
-    if (carry) {  // k == 63: the root
+    if (carry) {  // the last stage: the root
 #pragma unroll
-      for (int ct = 0; ct < 4; ++ct) res[ct] = cur[ct];
+      for (int c = 0; c < 4; ++c) res[c] = cur[c];
     }
-    if (k + 1 < 64) stage(buf ^ 1);
+    if (st + 1 < NST) stage(s_st + ((st + 1) & 1) * P::stage);
   }
-  const int g = kk, n = m;
   if constexpr (GLU) {
     // the up waves hand their values to the gate waves of the same rows
     __syncthreads();
-    float* s_up = &s_w[0][0];  // [2 tiles][4 ct][64 lanes][4]: 2,048 of the 2 x 64 x LS floats
-    if (wave >= 2)
+    float* s_up = s_st;  // [NW / 2 waves][4 tiles][64 lanes][4]
+    constexpr int GW = NW / 4;
+    if (wn >= GW)
 #pragma unroll
-      for (int ct = 0; ct < 4; ++ct) *(v4f*)(s_up + (((wave & 1) * 4 + ct) * 64 + lane) * 4) = res[ct];
+      for (int c = 0; c < 4; ++c) *(v4f*)(s_up + (((wave - 2 * GW) * 4 + c) * 64 + lane) * 4) = res[c];
     __syncthreads();
-    if (wave >= 2) return;
+    if (wn >= GW) return;
 #pragma unroll
-    for (int ct = 0; ct < 4; ++ct) {
-      const int t = s0 + 16 * ct + n;
-      if (t >= S) continue;
-      const v4f u = *(const v4f*)(s_up + (((wave & 1) * 4 + ct) * 64 + lane) * 4);
-      float v[4];
+    for (int c = 0; c < 4; ++c) {
+      const v4f u = *(const v4f*)(s_up + ((wave * 4 + c) * 64 + lane) * 4);
 #pragma unroll
-      for (int q = 0; q < 4; ++q) v[q] = dev_swiglu(res[ct][q], u[q]);
-      pf_store4(PF_EPI_STORE, out, N, t, 32 * blockIdx.x + 16 * (wave & 1) + 4 * g, v, nullptr);
+      for (int q = 0; q < 4; ++q) res[c][q] = dev_swiglu(res[c][q], u[q]);
     }
-  } else {
+  }
 #pragma unroll
-    for (int ct = 0; ct < 4; ++ct) {
-      const int t = s0 + 16 * ct + n;
-      if (t >= S) continue;
-      const float v[4] = {res[ct][0], res[ct][1], res[ct][2], res[ct][3]};
-      pf_store4(epi, out, N, t, 64 * blockIdx.x + 16 * wave + 4 * g, v, bias);
-    }
+  for (int c = 0; c < 4; ++c) {
+    const int t = s0 + 32 * ws + 16 * (c & 1) + m, n = nrow + 32 * wn + 16 * (c >> 1) + 4 * kk;
+    if (t >= S || n >= N) continue;
+    const float v[4] = {res[c][0], res[c][1], res[c][2], res[c][3]};
+    pf_store4(GLU ? (int)PF_EPI_STORE : epi, out, N, t, n, v, bias);
   }
 }
 
@@ -415,11 +451,20 @@ void launch_pf_gemm_wt(hipStream_t s, int wtype, int epi, const uint8_t* w, cons
   }
   const bool f32 = wtype == MTG_TYPE_F32;
   const void* xa = f32 ? (const void*)act.f32 : (const void*)act.f16h;
-#define MTG_PF_F16(G, L)                                                                                       \
-  if (f32)                                                                                                     \
-    hipLaunchKernelGGL((k_pf_gemm_f16<G, L, true>), grid, dim3(256), 0, s, w, w2, N, xa, S, out, epi, bias); \
-  else                                                                                                         \
-    hipLaunchKernelGGL((k_pf_gemm_f16<G, L, false>), grid, dim3(256), 0, s, w, w2, N, xa, S, out, epi, bias)
+  // eight waves (128 weight rows) once every CU gets a workgroup, else four: N 1,024, K 3,072,
+  // 2,048 rows 130 us with 256 workgroups of eight, 1,819 rows 130 us with 464 of four
+  const int wide_n = glu ? N / 64 : N / 128;
+  const bool wide = (size_t)wide_n * grid.y >= 256;
+  const dim3 wgrid((unsigned)((glu ? 2 * N : N) + 127) / 128, grid.y);
+#define MTG_PF_F16_W(G, L, F, NW, GRID) \
+  hipLaunchKernelGGL((k_pf_gemm_f16<G, L, F, NW>), GRID, dim3(64 * NW), (PfF16<L, NW>::bytes), s, w, w2, N, xa, S, out, epi, bias)
+#define MTG_PF_F16(G, L)                             \
+  do {                                               \
+    if (f32 && wide) MTG_PF_F16_W(G, L, true, 8, wgrid);  \
+    else if (f32) MTG_PF_F16_W(G, L, true, 4, grid);      \
+    else if (wide) MTG_PF_F16_W(G, L, false, 8, wgrid);   \
+    else MTG_PF_F16_W(G, L, false, 4, grid);              \
+  } while (0)
 #define MTG_PF_F16_K(G)                        \
   switch (K) {                                 \
     case 1024: MTG_PF_F16(G, 16); break;       \
@@ -431,6 +476,26 @@ void launch_pf_gemm_wt(hipStream_t s, int wtype, int epi, const uint8_t* w, cons
   else { MTG_PF_F16_K(false); }
 #undef MTG_PF_F16_K
 #undef MTG_PF_F16
+#undef MTG_PF_F16_W
+}
+
+hipError_t prepare_kernels_pf_wt() {
+  hipError_t e = hipSuccess;
+#define MTG_PF_LDS(G, L, F)                                                                                      \
+  if (e == hipSuccess)                                                                                           \
+    e = hipFuncSetAttribute((const void*)k_pf_gemm_f16<G, L, F, 8>, hipFuncAttributeMaxDynamicSharedMemorySize,  \
+                            (int)PfF16<L, 8>::bytes);                                                            \
+  if (e == hipSuccess)                                                                                           \
+    e = hipFuncSetAttribute((const void*)k_pf_gemm_f16<G, L, F, 4>, hipFuncAttributeMaxDynamicSharedMemorySize,  \
+                            (int)PfF16<L, 4>::bytes);
+#define MTG_PF_LDS_K(G, F) MTG_PF_LDS(G, 16, F) MTG_PF_LDS(G, 32, F) MTG_PF_LDS(G, 48, F) MTG_PF_LDS(G, 64, F)
+  MTG_PF_LDS_K(false, false)
+  MTG_PF_LDS_K(false, true)
+  MTG_PF_LDS_K(true, false)
+  MTG_PF_LDS_K(true, true)
+#undef MTG_PF_LDS_K
+#undef MTG_PF_LDS
+  return e;
 }
 
 int pf_gemm_wt_supported(int wtype, int K) {

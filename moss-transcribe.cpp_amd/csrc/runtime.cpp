@@ -252,6 +252,7 @@ int Ctx::init(const mtg_model_desc* d, int max_seq_in, int kv_type_in) {
     return fail(MTG_ERR_NOMEM, "step buffers");
   if ((rc = check(prepare_kernels(), "kernel attributes"))) return rc;
   if ((rc = check(prepare_kernels_wt(), "kernel attributes"))) return rc;
+  if ((rc = check(prepare_kernels_pf_wt(), "kernel attributes"))) return rc;
   if ((rc = init_step_kernel())) return rc;
   return check(hipDeviceSynchronize(), "init");
 }
