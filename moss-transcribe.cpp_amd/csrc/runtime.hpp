@@ -86,6 +86,11 @@ struct Ctx {
     // f16 / q4_K weights: the attention output rows and the GEMM activation
     float* o = nullptr;
     WtAct wact{};
+    // prompts of several blocks: a second set of input and hidden rows, and the stream
+    // that copies one set while the other block computes
+    float *x2 = nullptr, *hid2 = nullptr;
+    hipStream_t copy = nullptr;
+    hipEvent_t up[2] = {}, done[2] = {};
   } pf;
   bool prefill_fast_enabled = true;
   double last_prefill_ms = 0.0;  // device time of the last prefill (HIP events)
@@ -117,6 +122,8 @@ struct Ctx {
   // reset + S prompt rows; the block path when the weights are q8_0 and the
   // context fits the prefill attention, else verify-size appends
   int prefill(const float* embeds, int S, float* hidden_out);
+  template <class Block>
+  int prefill_pipeline(const float* embeds, int S, float* hidden_out, Block&& block);
   int prefill_blocks(const float* embeds, int S, float* hidden_out);
   int prefill_blocks_wt(const float* embeds, int S, float* hidden_out);
   int logits_of(const float* hidden, int T, float* logits_out);
