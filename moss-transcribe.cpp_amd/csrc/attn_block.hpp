@@ -44,10 +44,10 @@ struct AttnBlockArgs {
   const uint8_t* v;
   size_t head_bytes;
   int key_bytes;
-  int q_stride;         // floats
+  int q_stride, out_stride;  // floats
   int group;            // q heads per kv head (causal)
   int past, S, kvlen;   // rows 0 .. S - 1 at positions past + row; kvlen keys
-  float* out;           // f32 rows [row][q_stride], or
+  float* out;           // f32 rows [row][out_stride], or
   int8_t* ocodes;       // q8_0 codes and scales of rows of q_stride (q8_rows_code, q8_rows_scale)
   float* oscales;
 };
@@ -118,7 +118,7 @@ struct AbPiece {
 // positions past + row. Else: rows r0 + 16 u .. of head blockIdx.x, every key.
 // OUTQ: q8_0 codes and scales (HD == 128), else f32 rows.
 template <int HD, int KVH, bool CAUSAL, bool OUTQ>
-__global__ void __launch_bounds__(256, 2) k_attn_block(const AttnBlockArgs A) {
+__global__ void __launch_bounds__(256, HD == 64 ? 3 : 2) k_attn_block(const AttnBlockArgs A) {
   using Lds = AbLds<HD>;
   constexpr int NDT = HD / 16, NS = HD / 4, ES = KVH ? 2 : 4;
   extern __shared__ float ab_lds[];
@@ -578,7 +578,7 @@ __global__ void __launch_bounds__(256, 2) k_attn_block(const AttnBlockArgs A) {
   } else {
     if (orow >= A.S) return;
     const int d0 = (wave >> 1) * (NDT / 2);  // half of the dt tiles per wave
-    float* dst = A.out + (size_t)orow * A.q_stride + ooff;
+    float* dst = A.out + (size_t)orow * A.out_stride + ooff;
     float o[NDT / 2][4];
 #pragma unroll
     for (int dt = 0; dt < NDT / 2; ++dt) {

@@ -9,7 +9,8 @@
 //   layers     k_enc_ln: LayerNorm (mean and variance as double sums over 64
 //              lane partials, butterfly) -> q8_0 codes for the next GEMM;
 //              q / k / v / out / fc1 / fc2 on the block GEMM of the prefill
-//              (q8_0 weights x q8_0 activations, int8 MFMA) with bias, GELU or
+//              (q8_0 weights x q8_0 activations, int8 MFMA; q | k | v as one
+//              matrix: 1,500 rows 43 -> 27 us) with bias, GELU or
 //              residual epilogues; k_attn_block (attn_block.hpp): bidirectional
 //              attention on f32 MFMA, 32 query rows of one head per workgroup
 //   adaptor    merge consecutive rows (a view), fc1 + SiLU, fc2, LayerNorm
@@ -231,8 +232,8 @@ struct mtg_encoder {
   double last_ms = 0.0;
   int last_rows = 0;
   struct Layer {
-    float *attn_ln_w, *attn_ln_b, *q_b, *v_b, *o_b, *ffn_ln_w, *ffn_ln_b, *fc1_b, *fc2_b;
-    uint8_t *q_w, *k_w, *v_w, *o_w, *fc1_w, *fc2_w;
+    float *attn_ln_w, *attn_ln_b, *qkv_b, *o_b, *ffn_ln_w, *ffn_ln_b, *fc1_b, *fc2_b;
+    uint8_t *qkv_w, *o_w, *fc1_w, *fc2_w;  // q | k | v: one matrix of 3 d_model rows
   };
   std::vector<Layer> layers;
   float *conv1_w = nullptr, *conv1_b = nullptr, *conv2_w = nullptr, *conv2_b = nullptr, *pos = nullptr,
@@ -240,7 +241,7 @@ struct mtg_encoder {
   uint8_t *ad_fc1_w = nullptr, *ad_fc2_w = nullptr;
   float *ad_fc1_b = nullptr, *ad_fc2_b = nullptr, *ad_ln_w = nullptr, *ad_ln_b = nullptr;
   // activations
-  float *mel = nullptr, *c1 = nullptr, *x = nullptr, *q = nullptr, *k = nullptr, *v = nullptr, *a = nullptr,
+  float *mel = nullptr, *c1 = nullptr, *x = nullptr, *qkv = nullptr, *a = nullptr,
         *f = nullptr, *out_rows = nullptr, *in_rows = nullptr, *h1 = nullptr, *h2 = nullptr, *ad_out = nullptr;
   int8_t* codes = nullptr;
   float* scales = nullptr;
@@ -288,13 +289,13 @@ struct mtg_encoder {
     rc = check(hipMemcpy(d, src, n * 4, hipMemcpyHostToDevice), "upload");
     return d;
   }
-  uint8_t* up_q8(const void* src, int n, int kk, uint8_t* staging, int& rc) {
+  uint8_t* up_q8(const void* src, int n, int kk, uint8_t* staging, int& rc, uint8_t* at) {
     if (rc) return nullptr;
     if (!src) {
       rc = fail(MTG_ERR_INVALID, "a tensor pointer is NULL");
       return nullptr;
     }
-    uint8_t* d = (uint8_t*)dalloc(q8_tiles_bytes(n, kk));
+    uint8_t* d = at ? at : (uint8_t*)dalloc(q8_tiles_bytes(n, kk));
     if (!d) {
       rc = fail(MTG_ERR_NOMEM, "device memory");
       return nullptr;
@@ -306,18 +307,24 @@ struct mtg_encoder {
     rc = check(hipStreamSynchronize(stream), "retile");
     return d;
   }
-  // an n x kk matrix: q8_0 re-tiled for the int8 MFMA GEMM, f16 / f32 / q4_K as they are
-  uint8_t* up_w(const void* src, int n, int kk, uint8_t* staging, int& rc) {
-    if (wtype == MTG_TYPE_Q8_0) return up_q8(src, n, kk, staging, rc);
+  // bytes of an n x kk matrix on the device
+  size_t w_bytes(int n, int kk) const {
+    if (wtype == MTG_TYPE_Q8_0) return q8_tiles_bytes(n, kk);
+    return (size_t)n * (wtype == MTG_TYPE_F16   ? (size_t)kk * 2
+                        : wtype == MTG_TYPE_F32 ? (size_t)kk * 4
+                                                : (size_t)(kk / 256) * 144);
+  }
+  // an n x kk matrix: q8_0 re-tiled for the int8 MFMA GEMM, f16 / f32 / q4_K as they are;
+  // into memory of its own, or to `at`
+  uint8_t* up_w(const void* src, int n, int kk, uint8_t* staging, int& rc, uint8_t* at = nullptr) {
+    if (wtype == MTG_TYPE_Q8_0) return up_q8(src, n, kk, staging, rc, at);
     if (rc) return nullptr;
     if (!src) {
       rc = fail(MTG_ERR_INVALID, "a tensor pointer is NULL");
       return nullptr;
     }
-    const size_t bytes = (size_t)n * (wtype == MTG_TYPE_F16   ? (size_t)kk * 2
-                                      : wtype == MTG_TYPE_F32 ? (size_t)kk * 4
-                                                              : (size_t)(kk / 256) * 144);
-    uint8_t* d = (uint8_t*)dalloc(bytes);
+    const size_t bytes = w_bytes(n, kk);
+    uint8_t* d = at ? at : (uint8_t*)dalloc(bytes);
     if (!d) {
       rc = fail(MTG_ERR_NOMEM, "device memory");
       return nullptr;
@@ -387,17 +394,27 @@ int mtg_encoder_create(const mtg_encoder_desc* d, mtg_encoder** out) {
   e->pos = e->up_f(d->pos_embd, (size_t)R * D, rc);
   e->ln_post_w = e->up_f(d->ln_post_w, D, rc);
   e->ln_post_b = e->up_f(d->ln_post_b, D, rc);
+  std::vector<float> qkv_b((size_t)3 * D, 0.0f);
   for (int l = 0; l < hp.n_layers && !rc; ++l) {
     const mtg_encoder_layer& s = d->layers[l];
     mtg_encoder::Layer L{};
     L.attn_ln_w = e->up_f(s.attn_ln_w, D, rc);
     L.attn_ln_b = e->up_f(s.attn_ln_b, D, rc);
-    L.q_w = e->up_w(s.q_w, D, D, staging, rc);
-    L.k_w = e->up_w(s.k_w, D, D, staging, rc);
-    L.v_w = e->up_w(s.v_w, D, D, staging, rc);
+    const size_t part = e->w_bytes(D, D);
+    L.qkv_w = rc ? nullptr : (uint8_t*)e->dalloc(3 * part);
+    if (!rc && !L.qkv_w) rc = e->fail(MTG_ERR_NOMEM, "device memory");
+    e->up_w(s.q_w, D, D, staging, rc, L.qkv_w);
+    e->up_w(s.k_w, D, D, staging, rc, L.qkv_w + part);
+    e->up_w(s.v_w, D, D, staging, rc, L.qkv_w + 2 * part);
     L.o_w = e->up_w(s.o_w, D, D, staging, rc);
-    L.q_b = e->up_f(s.q_b, D, rc);
-    L.v_b = e->up_f(s.v_b, D, rc);
+    // k has no bias: + 0 leaves its sums as they are (their chains start at +0, so none is
+    // -0 unless every f32 product of one underflows)
+    if (!rc && (!s.q_b || !s.v_b)) rc = e->fail(MTG_ERR_INVALID, "a tensor pointer is NULL");
+    if (!rc) {
+      std::copy(s.q_b, s.q_b + D, qkv_b.begin());
+      std::copy(s.v_b, s.v_b + D, qkv_b.begin() + 2 * D);
+    }
+    L.qkv_b = e->up_f(qkv_b.data(), 3 * (size_t)D, rc);
     L.o_b = e->up_f(s.o_b, D, rc);
     L.ffn_ln_w = e->up_f(s.ffn_ln_w, D, rc);
     L.ffn_ln_b = e->up_f(s.ffn_ln_b, D, rc);
@@ -418,9 +435,7 @@ int mtg_encoder_create(const mtg_encoder_desc* d, mtg_encoder** out) {
     e->mel = (float*)e->dalloc((size_t)M * NF * 4);
     e->c1 = (float*)e->dalloc((size_t)D * NF * 4);
     e->x = (float*)e->dalloc(RD * 4);
-    e->q = (float*)e->dalloc(RD * 4);
-    e->k = (float*)e->dalloc(RD * 4);
-    e->v = (float*)e->dalloc(RD * 4);
+    e->qkv = (float*)e->dalloc(3 * RD * 4);
     e->a = (float*)e->dalloc(RD * 4);
     e->f = (float*)e->dalloc((size_t)R * F * 4);
     e->out_rows = (float*)e->dalloc(RD * 4);
@@ -449,7 +464,7 @@ int mtg_encoder_create(const mtg_encoder_desc* d, mtg_encoder** out) {
       e->xn = (float*)e->dalloc(RD * 4);
       if (!e->xn) rc = e->fail(MTG_ERR_NOMEM, "device memory");
     }
-    if (!e->mel || !e->c1 || !e->x || !e->q || !e->k || !e->v || !e->a || !e->f || !e->out_rows || !e->in_rows ||
+    if (!e->mel || !e->c1 || !e->x || !e->qkv || !e->a || !e->f || !e->out_rows || !e->in_rows ||
         !e->h1 || !e->h2 || !e->ad_out || !e->codes || !e->scales)
       rc = e->fail(MTG_ERR_NOMEM, "device memory");
   }
@@ -482,19 +497,18 @@ int mtg_encoder_encode(mtg_encoder* e, const float* mel, float* out, int32_t* ro
                      e->conv2_w, e->conv2_b, e->c1, D, NF, D, e->pos, e->x);
   const dim3 agrid((unsigned)hp.n_heads, (unsigned)((R + 31) / 32));
   AttnBlockArgs attn{};
-  attn.q = e->q;
-  attn.k = (const uint8_t*)e->k;
-  attn.v = (const uint8_t*)e->v;
+  attn.q = e->qkv;
+  attn.k = (const uint8_t*)(e->qkv + D);
+  attn.v = (const uint8_t*)(e->qkv + 2 * D);
   attn.head_bytes = kEncHd * 4;
-  attn.key_bytes = D * 4;
-  attn.q_stride = D;
+  attn.key_bytes = 3 * D * 4;
+  attn.q_stride = 3 * D;
+  attn.out_stride = D;
   attn.S = attn.kvlen = R;
   attn.out = e->a;
   for (const mtg_encoder::Layer& L : e->layers) {
     e->ln(e->x, R, L.attn_ln_w, L.attn_ln_b, 1e-5f, true, nullptr);
-    e->gemm(PF_EPI_BIAS, L.q_w, D, D, R, e->q, L.q_b);
-    e->gemm(PF_EPI_STORE, L.k_w, D, D, R, e->k, nullptr);
-    e->gemm(PF_EPI_BIAS, L.v_w, D, D, R, e->v, L.v_b);
+    e->gemm(PF_EPI_BIAS, L.qkv_w, 3 * D, D, R, e->qkv, L.qkv_b);
     hipLaunchKernelGGL((k_attn_block<kEncHd, 0, false, false>), agrid, dim3(256), AbLds<kEncHd>::bytes, s, attn);
     e->quant(e->a, R, D);
     e->gemm(PF_EPI_BIAS_RESID, L.o_w, D, D, R, e->x, L.o_b);

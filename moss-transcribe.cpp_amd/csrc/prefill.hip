@@ -378,7 +378,7 @@ void launch_pf_attn(hipStream_t s, const float* q, int n_heads, int n_kv_heads, 
   a.v = (const uint8_t*)kv.v;
   a.head_bytes = (size_t)kv.max_seq * kHeadDim * es;
   a.key_bytes = kHeadDim * es;
-  a.q_stride = n_heads * kHeadDim;
+  a.q_stride = a.out_stride = n_heads * kHeadDim;
   a.group = n_heads / n_kv_heads;
   a.past = past0;
   a.S = S;
