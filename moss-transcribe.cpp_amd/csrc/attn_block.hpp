@@ -20,12 +20,12 @@
 // A workgroup takes 2 query tiles of 16; its four waves take chunks c = wave mod 4.
 // Every chunk's (l_c, O_c) is computed independently; the running (L, O) travels
 // from wave to wave through LDS in chunk order (the merge is 1 / 16 of the work).
-// Two workgroups per CU, two waves per SIMD.
+// Two workgroups per CU, two waves per SIMD (head_dim 64: three).
 // Measured against two exact passes with K and V^T staged by the whole workgroup:
-// 1,600 rows, f32 cache 289 -> 200 us per layer (the MFMAs alone: 69 us; the rest is
+// 1,600 rows, f32 cache 289 -> 205 us per layer (the MFMAs alone: 69 us; the rest is
 // the estimates' reads of K at the start, vector work and the uneven causal blocks);
 // 2,048 rows after 14,336, f16 cache 3.84 -> 2.6 ms (1.64 ms); the
-// encoder's 1,500 rows x 16 heads 202 -> 161 us (60 us).
+// encoder's 1,500 rows x 16 heads 202 -> 153 us (60 us).
 #pragma once
 
 #include <hip/hip_fp16.h>

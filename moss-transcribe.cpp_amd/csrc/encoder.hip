@@ -10,7 +10,7 @@
 //              lane partials, butterfly) -> q8_0 codes for the next GEMM;
 //              q / k / v / out / fc1 / fc2 on the block GEMM of the prefill
 //              (q8_0 weights x q8_0 activations, int8 MFMA; q | k | v as one
-//              matrix: 1,500 rows 43 -> 27 us) with bias, GELU or
+//              matrix: 1,500 rows 43 -> 32 us) with bias, GELU or
 //              residual epilogues; k_attn_block (attn_block.hpp): bidirectional
 //              attention on f32 MFMA, 32 query rows of one head per workgroup
 //   adaptor    merge consecutive rows (a view), fc1 + SiLU, fc2, LayerNorm
