@@ -357,7 +357,8 @@ void mtg_q8_free(mtg_q8_packed* p);
  * (reference: PackedQ8::round_trip_exact, src/cpu_q8.hpp:17). */
 int mtg_q8_unpack(const mtg_q8_packed* p, void* blocks);
 /* y_dev[t][n] = q8_0 dot of the packed rows with x_dev[t][:] (T x K floats,
- * quantized to q8_0 per 32-block on the device), T in 1..MTG_MAX_BATCH. */
+ * quantized to q8_0 per 32-block on the device), T in 1..MTG_MAX_BATCH. y_dev may
+ * overlap x_dev (x is read before y is written, on a slower path). */
 int mtg_q8_mul_mat_dev(const mtg_q8_packed* w, const float* x_dev, int32_t T, float* y_dev);
 
 /* mtg_q8_mul_mat_dev without any allocation (no counterpart in the reference;

@@ -64,8 +64,9 @@ CPP_TESTS = os.path.join(ROOT, "tests", "cpp")
 
 
 def build_cpp_tests():
-    """The C++ test drivers of the reference-named interface (tests/cpp), linked
-    against libmtg.so; binaries go to tests/cpp/bin (git-ignored)."""
+    """The C++ test drivers (tests/cpp), linked against libmtg.so; binaries go to
+    tests/cpp/bin (git-ignored). -rdynamic: fake_hip.hpp's symbols stand in for the HIP
+    runtime's in the programs that include it."""
     out_dir = os.path.join(CPP_TESTS, "bin")
     os.makedirs(out_dir, exist_ok=True)
     outs = []
@@ -73,7 +74,7 @@ def build_cpp_tests():
         if not name.endswith(".cpp"):
             continue
         exe = os.path.join(out_dir, name[:-4])
-        _run(["g++", "-std=c++17", "-O1", "-Wall", "-I", os.path.join(ROOT, "include"),
+        _run(["g++", "-std=c++17", "-O1", "-Wall", "-rdynamic", "-I", os.path.join(ROOT, "include"),
               os.path.join(CPP_TESTS, name), "-o", exe, "-L", PKG, "-lmtg",
               "-Wl,-rpath," + PKG, "-Wl,-rpath-link,/opt/rocm/lib"])
         outs.append(exe)

@@ -950,6 +950,9 @@ bool launch_mul_mat(hipStream_t s, const uint8_t* w, int n, int k, const float* 
   const int bps = k / kPairK, G = (T + 7) / 8, tiles = n / 16;
   const size_t lds = mul_mat_panel_bytes(bps, G);
   if (lds > (size_t)kMulMatLds || ((uintptr_t)x | (uintptr_t)y) % 16) return false;
+  // Its workgroups convert x each for themselves while others store y, in no order: only
+  // the general path, which has x in a panel before its product starts, may overwrite x.
+  if ((uintptr_t)x < (uintptr_t)(y + (size_t)T * n) && (uintptr_t)y < (uintptr_t)(x + (size_t)T * k)) return false;
   // A workgroup per tile while converting the panel that often is cheap; else 1,024
   // workgroups walk the tiles, which streams as fast as the general path only with four
   // panels to a CU (K 4,096, 16 rows, N 16,384: 56 us against the general path's 47; 8

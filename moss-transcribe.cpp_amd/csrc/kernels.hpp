@@ -55,10 +55,11 @@ void launch_embed(hipStream_t s, const StepDesc* desc, const uint8_t* embd_tiles
 // normed_out (nullable) receives the f32 normalized rows.
 void launch_norm_quant(hipStream_t s, const StepDesc* desc, const float* src, int K,
                        const float* gain, float eps, Panel panel, float* normed_out);
-// out[t][n] = W . x[t] for all rows of a packed matrix (epilogue: store).
 // y = x (T rows, q8_0 on the device) times a packed q8_0 matrix, one launch; false where
-// its LDS panel or the pointers' alignment (16 bytes) does not allow it.
+// its LDS panel, the pointers' alignment (16 bytes) or an overlap of x and y does not
+// allow it.
 bool launch_mul_mat(hipStream_t s, const uint8_t* w, int n, int k, const float* x, int T, float* y);
+// out[t][n] = W . x[t] for all rows of a packed matrix (epilogue: store).
 void launch_gemm_store(hipStream_t s, int G, const StepDesc* desc, const uint8_t* w, int n, int k,
                        Panel x, float* out);
 // x[t][n] += W . act[t] (o-proj and down-proj with residual).

@@ -1,0 +1,59 @@
+// Which kernels mtg_q8_mul_mat_dev launches, on the fake HIP runtime: the one-launch
+// product where it may run, else the general path (conversion into a panel, then the
+// product). k_mul_mat's workgroups read every row of x for themselves while others
+// already store y, so operands that overlap belong on the general path, whose first
+// launch has converted all of x before the second one writes y.
+#include "fake_hip.hpp"
+
+#include <cstdio>
+#include <vector>
+
+#include "mtg_verify.h"
+
+static int failures = 0;
+static void expect(bool ok, const char* what, long a = 0, long b = 0) {
+  if (ok) return;
+  std::fprintf(stderr, "%s (%ld, %ld)\n", what, a, b);
+  ++failures;
+}
+
+struct Matrix {
+  mtg_q8_packed* w = nullptr;
+  Matrix(int k, int n) {
+    std::vector<uint8_t> raw((size_t)n * (k / 32) * 34, 0);
+    expect(mtg_q8_pack(raw.data(), k, n, &w) == MTG_OK, "pack", k, n);
+  }
+  ~Matrix() { mtg_q8_free(w); }
+};
+// 1: the one-launch kernel alone, 2: the general path alone
+static int route(const Matrix& m, const float* x, int T, float* y) {
+  fake::state().launches.clear();
+  expect(mtg_q8_mul_mat_dev(m.w, x, T, y) == MTG_OK, "product", T);
+  const int one = fake::count("k_mul_mat"), all = (int)fake::state().launches.size();
+  return one == 1 && all == 1 ? 1 : one == 0 && all == 2 ? 2 : -1;
+}
+
+static void overlap() {
+  const int k = 1024, n = 1024, other = 512;
+  Matrix square(k, n), narrow(k, other);
+  std::vector<float> buf(4 * 16 * 1024 + 4);
+  float* at = (float*)(((uintptr_t)buf.data() + 15) & ~(uintptr_t)15);
+  const int Ts[] = {1, 8, 9, 16};
+  for (int T : Ts) {
+    const int xs = T * k, ys = T * n, ns = T * other;
+    expect(route(square, at, T, at + xs) == 1, "y behind x", T);
+    expect(route(square, at + ys, T, at) == 1, "y ahead of x", T);
+    expect(route(square, at, T, at) == 2, "y is x", T);
+    expect(route(square, at, T, at + xs - 4) == 2, "y begins in x", T);
+    expect(route(square, at + ys - 4, T, at) == 2, "y ends in x", T);
+    expect(route(narrow, at, T, at + 4) == 2, "y inside x", T);
+    expect(route(narrow, at + ns, T, at) == 1, "narrow y ahead of x", T);
+    expect(route(narrow, at, T, at + xs) == 1, "narrow y behind x", T);
+  }
+}
+
+int main() {
+  overlap();
+  std::printf("{\"record\": \"mulMatRoute\", \"failures\": %d}\n", failures);
+  return failures ? 1 : 0;
+}

@@ -38,3 +38,9 @@ def test_cpp_speculative_gate_on_gpu():
 def test_erf_polynomials_round_as_the_series():
     rec = _run("test_erf_poly", 100)
     assert rec["differ"] == 0 and rec["floats"] > 17_000_000
+
+
+def test_product_alone_takes_the_kernels_it_may():
+    """csrc/kernels.hip launch_mul_mat on the fake HIP runtime: x and y that overlap."""
+    rec = _run("test_mul_mat_route", 60)
+    assert rec == {"record": "mulMatRoute", "failures": 0}

@@ -38,3 +38,29 @@ def test_mul_mat_edges(k, n, T, shift):
     y = yd.cpu().numpy()
     assert np.array_equal(y[shift:shift + T * n].reshape(T, n), ref)
     assert (y[:shift] == 7.0).all() and (y[shift + T * n:] == 7.0).all()
+
+
+@pytest.mark.parametrize("k,n,T,y_at", [(1024, 1024, 1, 0), (1024, 1024, 16, 0), (256, 256, 8, 255), (256, 256, 9, -255),
+                                        (1024, 512, 16, 64)])
+def test_mul_mat_over_its_own_input(k, n, T, y_at):
+    """y over x, or y_at floats away from its start: x is read before y is written."""
+    print("mul_mat over x: k %d n %d T %d y at x %+d" % (k, n, T, y_at), flush=True)
+    rng = np.random.default_rng(k + n + T)
+    w = (rng.standard_normal((n, k)) * 0.02).astype(np.float32)
+    raw = np.empty(n * (k // 32) * 34, np.uint8)
+    mtg.lib().mtg_quantize_q8_0_weight(mtg.ptr(w), n * k, mtg.ptr(raw))
+    x = rng.standard_normal((T, k)).astype(np.float32)
+    ref = oracle_py.mul_mat(mtg.TYPE_Q8_0, raw, k, n, x)
+    packed = ctypes.c_void_p()
+    assert mtg.lib().mtg_q8_pack(mtg.ptr(raw), k, n, ctypes.byref(packed)) == 0
+    buf = torch.full((T * max(k, n) + 512,), 7.0, device="cuda")
+    xo, yo = 256, 256 + y_at
+    buf[xo:xo + T * k] = torch.from_numpy(x.reshape(-1)).cuda()
+    torch.cuda.synchronize()
+    rc = mtg.lib().mtg_q8_mul_mat_dev(packed, ctypes.c_void_p(buf.data_ptr() + 4 * xo), T,
+                                      ctypes.c_void_p(buf.data_ptr() + 4 * yo))
+    mtg.lib().mtg_q8_free(packed)
+    assert rc == 0
+    got = buf.cpu().numpy()
+    assert np.array_equal(got[yo:yo + T * n].reshape(T, n), ref)
+    assert (got[:min(xo, yo)] == 7.0).all() and (got[max(xo + T * k, yo + T * n):] == 7.0).all()
