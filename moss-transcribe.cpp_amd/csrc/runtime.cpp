@@ -70,7 +70,10 @@ int Ctx::check(hipError_t e, const char* what) {
 
 void* Ctx::dalloc(size_t bytes, bool zero) {
   void* p = nullptr;
-  if (hipMalloc(&p, bytes ? bytes : 16) != hipSuccess) return nullptr;
+  if (hipMalloc(&p, bytes ? bytes : 16) != hipSuccess) {
+    (void)hipGetLastError();  // the caller's to report: no later launch check finds it
+    return nullptr;
+  }
   allocations.push_back(p);
   if (zero && hipMemset(p, 0, bytes ? bytes : 16) != hipSuccess) return nullptr;
   return p;
@@ -695,7 +698,8 @@ int Ctx::prefill_blocks(const float* embeds, int S, float* hidden_out) {
 // stream. With several blocks their rows travel on a second stream: while a block
 // computes, the previous block's hidden rows come back and the next one's inputs go out.
 // Copies of pageable memory hold the host, so on one stream every block boundary left the
-// device idle for both (16,384 rows: about 7 of 65 ms).
+// device idle for both (16,384 rows: about 7 of 65 ms). Without memory for the second set
+// of rows (16.8 MB) the blocks do run that way.
 template <class Block>
 int Ctx::prefill_pipeline(const float* embeds, int S, float* hidden_out, Block&& block) {
   const int H = hp.hidden, R = kPfRows, nb = (S + R - 1) / R;
@@ -709,11 +713,11 @@ int Ctx::prefill_pipeline(const float* embeds, int S, float* hidden_out, Block&&
   if (nb > 1) {
     if (!pf.copy && (rc = check(hipStreamCreateWithFlags(&pf.copy, hipStreamNonBlocking), "stream"))) return rc;
     if (!pf.x2) pf.x2 = (float*)dalloc((size_t)R * H * 4, false);
-    if (!pf.hid2) pf.hid2 = (float*)dalloc((size_t)R * H * 4, false);
-    if (!pf.x2 || !pf.hid2) return fail(MTG_ERR_NOMEM, "prefill buffers");
+    if (pf.x2 && !pf.hid2) pf.hid2 = (float*)dalloc((size_t)R * H * 4, false);
   }
-  hipStream_t s = stream, cs = nb > 1 ? pf.copy : stream;
-  float *const x[2] = {pf.x, pf.x2}, *const hid[2] = {pf.hid, pf.hid2};
+  const bool overlap = nb > 1 && pf.x2 && pf.hid2;
+  hipStream_t s = stream, cs = overlap ? pf.copy : stream;
+  float *const x[2] = {pf.x, overlap ? pf.x2 : pf.x}, *const hid[2] = {pf.hid, overlap ? pf.hid2 : pf.hid};
   auto rows = [&](int b) { return std::min(R, S - b * R); };
   auto up = [&](int b) {
     const int e = check(hipMemcpyAsync(x[b & 1], embeds + (size_t)b * R * H, (size_t)rows(b) * H * 4,
@@ -734,10 +738,10 @@ int Ctx::prefill_pipeline(const float* embeds, int S, float* hidden_out, Block&&
     block(b * R, rows(b), x[b & 1], hid[b & 1]);
     if ((rc = check(hipGetLastError(), "prefill launch"))) break;
     if ((rc = check(hipEventRecord(pf.done[b & 1], s), "event"))) break;
-    if (b > 0 && (rc = down(b - 1))) break;
+    if (overlap ? b > 0 && (rc = down(b - 1)) : (rc = down(b))) break;
     if (b + 1 < nb) rc = up(b + 1);
   }
-  if (!rc) rc = down(nb - 1);
+  if (!rc && overlap) rc = down(nb - 1);
   if (!rc) rc = check(hipEventRecord(ev_stop, cs), "event");
   // both streams are idle before the call returns, also after an error
   const int e1 = check(hipStreamSynchronize(cs), "prefill"), e2 = check(hipStreamSynchronize(s), "prefill");

@@ -44,3 +44,10 @@ def test_product_alone_takes_the_kernels_it_may():
     """csrc/kernels.hip launch_mul_mat on the fake HIP runtime: x and y that overlap."""
     rec = _run("test_mul_mat_route", 60)
     assert rec == {"record": "mulMatRoute", "failures": 0}
+
+
+def test_prompts_of_several_blocks_and_their_buffers():
+    """The prefill's streams, copies and buffers on the fake HIP runtime, with and
+    without memory for the second set of rows."""
+    rec = _run("test_prefill_buffers", 60)
+    assert rec == {"record": "prefillBuffers", "failures": 0}

@@ -119,3 +119,26 @@ def test_full_size_prefill_paths_and_time(cfg_id):
     a.close()
     b.close()
     model.close()
+
+
+@pytest.mark.parametrize("wtype", [mtg.TYPE_Q8_0, mtg.TYPE_F16], ids=["q8_0", "f16"])
+@pytest.mark.parametrize("S", [2049, 4100])
+def test_several_blocks_without_hidden_rows(S, wtype):
+    """A program that only fills the cache (hidden_out NULL): no rows come back between
+    the blocks, and the cache is the one of a prompt whose hidden rows do."""
+    print("blocks without hidden rows: S=%d weights %d" % (S, wtype), flush=True)
+    model = mtg.SynthModel(wtype, seed=45, std=0.02, gain_jitter=0.05, n_layers=2, vocab=256)
+    rows = mtg.normal(46, 0, S * 1024).reshape(S, 1024) * np.float32(0.03)
+    a, b = mtg.Decoder(model, S + 8), mtg.Decoder(model, S + 8)
+    b.prefill_mode(False)
+    b.prefill(rows)
+    row = rows[:1]
+    want = b.append(row)
+    for hidden in (False, True, False):
+        a.prefill(rows, want_hidden=hidden)
+        for x, y, what in zip(a.kv_read(S), b.kv_read(S), "kv"):
+            _same(x, y, "%s cache, hidden %s" % (what, hidden))
+        _same(a.append(row), want, "the next row, hidden %s" % hidden)
+    a.close()
+    b.close()
+    model.close()
