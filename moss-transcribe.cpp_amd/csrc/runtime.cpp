@@ -654,6 +654,23 @@ int Ctx::prefill(const float* embeds, int S, float* hidden_out) {
   return MTG_OK;
 }
 
+// A prefill buffer of n elements, made where it is not there yet: a prompt that ran out
+// of memory half way makes the missing ones when it is repeated.
+template <class T>
+bool Ctx::pf_buffer(T*& p, size_t n) {
+  if (!p) p = (T*)dalloc(n * sizeof(T), false);
+  return p != nullptr;
+}
+
+// the buffers of a block that every weight type has
+bool Ctx::prefill_rows_memory() {
+  const size_t R = kPfRows, H = hp.hidden, QN = (size_t)hp.n_heads * hp.head_dim, F = hp.intermediate;
+  const size_t NQKV = QN + 2 * (size_t)hp.n_kv_heads * hp.head_dim, KM = std::max(H, std::max(QN, F));
+  return pf_buffer(pf.x, R * H) && pf_buffer(pf.qkv, R * NQKV) && pf_buffer(pf.q, R * QN) &&
+         pf_buffer(pf.act, R * F) && pf_buffer(pf.hid, R * H) && pf_buffer(pf.codes, R * KM) &&
+         pf_buffer(pf.scales, R * (KM / 32));
+}
+
 // The prompt in blocks of kPfRows rows: per layer RMSNorm + q8_0 conversion, the
 // fused q|k|v GEMM, q/k norm + RoPE + KV append, causal attention over the cache,
 // o-proj + residual, RMSNorm, gate/up + SwiGLU, q8_0, down + residual; each
@@ -662,19 +679,7 @@ int Ctx::prefill_blocks(const float* embeds, int S, float* hidden_out) {
   const int H = hp.hidden, NH = hp.n_heads, NKV = hp.n_kv_heads, D = hp.head_dim;
   const int QN = NH * D, KN = NKV * D, NQKV = QN + 2 * KN, F = hp.intermediate;
   const float eps = hp.rms_eps;
-  const int R = kPfRows;
-  if (!pf.x) {
-    pf.x = (float*)dalloc((size_t)R * H * 4, false);
-    pf.qkv = (float*)dalloc((size_t)R * NQKV * 4, false);
-    pf.q = (float*)dalloc((size_t)R * QN * 4, false);
-    pf.act = (float*)dalloc((size_t)R * F * 4, false);
-    pf.hid = (float*)dalloc((size_t)R * H * 4, false);
-    const int KM = std::max(H, std::max(QN, F));
-    pf.codes = (int8_t*)dalloc((size_t)R * KM, false);
-    pf.scales = (float*)dalloc((size_t)R * (KM / 32) * 4, false);
-    if (!pf.x || !pf.qkv || !pf.q || !pf.act || !pf.hid || !pf.codes || !pf.scales)
-      return fail(MTG_ERR_NOMEM, "prefill buffers");
-  }
+  if (!prefill_rows_memory()) return fail(MTG_ERR_NOMEM, "prefill buffers");
   hipStream_t s = stream;
   return prefill_pipeline(embeds, S, hidden_out, [&](int c0, int n, float* x, float* hid) {
     for (int l = 0; l < hp.n_layers; ++l) {
@@ -712,10 +717,8 @@ int Ctx::prefill_pipeline(const float* embeds, int S, float* hidden_out, Block&&
   }
   if (nb > 1) {
     if (!pf.copy && (rc = check(hipStreamCreateWithFlags(&pf.copy, hipStreamNonBlocking), "stream"))) return rc;
-    if (!pf.x2) pf.x2 = (float*)dalloc((size_t)R * H * 4, false);
-    if (pf.x2 && !pf.hid2) pf.hid2 = (float*)dalloc((size_t)R * H * 4, false);
   }
-  const bool overlap = nb > 1 && pf.x2 && pf.hid2;
+  const bool overlap = nb > 1 && pf_buffer(pf.x2, (size_t)R * H) && pf_buffer(pf.hid2, (size_t)R * H);
   hipStream_t s = stream, cs = overlap ? pf.copy : stream;
   float *const x[2] = {pf.x, overlap ? pf.x2 : pf.x}, *const hid[2] = {pf.hid, overlap ? pf.hid2 : pf.hid};
   auto rows = [&](int b) { return std::min(R, S - b * R); };
@@ -762,32 +765,15 @@ int Ctx::prefill_blocks_wt(const float* embeds, int S, float* hidden_out) {
   const float eps = hp.rms_eps;
   const int R = kPfRows;
   const int KM = std::max(H, std::max(QN, F));
-  if (!pf.x) {
-    pf.x = (float*)dalloc((size_t)R * H * 4, false);
-    pf.qkv = (float*)dalloc((size_t)R * NQKV * 4, false);
-    pf.q = (float*)dalloc((size_t)R * QN * 4, false);
-    pf.act = (float*)dalloc((size_t)R * F * 4, false);
-    pf.hid = (float*)dalloc((size_t)R * H * 4, false);
-    pf.codes = (int8_t*)dalloc((size_t)R * KM, false);
-    pf.scales = (float*)dalloc((size_t)R * (KM / 32) * 4, false);
-    if (!pf.x || !pf.qkv || !pf.q || !pf.act || !pf.hid || !pf.codes || !pf.scales)
-      return fail(MTG_ERR_NOMEM, "prefill buffers");
-  }
-  if (!pf.o) {
-    pf.o = (float*)dalloc((size_t)R * QN * 4, false);
-    bool ok = true;
-    if (wtype == MTG_TYPE_F16) {
-      ok = (pf.wact.f16h = (uint16_t*)dalloc((size_t)R * KM * 2, false)) != nullptr;
-    } else if (wtype == MTG_TYPE_F32) {
-      ok = (pf.wact.f32 = (float*)dalloc((size_t)R * KM * 4, false)) != nullptr;
-    } else {
-      pf.wact.q8k.qs = (int8_t*)dalloc((size_t)R * KM, false);
-      pf.wact.q8k.d = (float*)dalloc((size_t)R * (KM / 256) * 4, false);
-      pf.wact.q8k.bsums = (int32_t*)dalloc((size_t)R * (KM / 16) * 4, false);
-      ok = pf.wact.q8k.qs && pf.wact.q8k.d && pf.wact.q8k.bsums;
-    }
-    if (!pf.o || !ok) return fail(MTG_ERR_NOMEM, "prefill buffers");
-  }
+  bool ok = prefill_rows_memory() && pf_buffer(pf.o, (size_t)R * QN);
+  if (wtype == MTG_TYPE_F16)
+    ok = ok && pf_buffer(pf.wact.f16h, (size_t)R * KM);
+  else if (wtype == MTG_TYPE_F32)
+    ok = ok && pf_buffer(pf.wact.f32, (size_t)R * KM);
+  else
+    ok = ok && pf_buffer(pf.wact.q8k.qs, (size_t)R * KM) && pf_buffer(pf.wact.q8k.d, (size_t)R * (KM / 256)) &&
+         pf_buffer(pf.wact.q8k.bsums, (size_t)R * (KM / 16));
+  if (!ok) return fail(MTG_ERR_NOMEM, "prefill buffers");
   hipStream_t s = stream;
   const WtAct& A = pf.wact;
   return prefill_pipeline(embeds, S, hidden_out, [&](int c0, int n, float* x, float* hid) {

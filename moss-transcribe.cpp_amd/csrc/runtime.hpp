@@ -122,6 +122,9 @@ struct Ctx {
   // reset + S prompt rows; the block path when the weights are q8_0 and the
   // context fits the prefill attention, else verify-size appends
   int prefill(const float* embeds, int S, float* hidden_out);
+  template <class T>
+  bool pf_buffer(T*& p, size_t n);
+  bool prefill_rows_memory();
   template <class Block>
   int prefill_pipeline(const float* embeds, int S, float* hidden_out, Block&& block);
   int prefill_blocks(const float* embeds, int S, float* hidden_out);

@@ -79,6 +79,27 @@ int main() {
       prompt(ctx, 5000, true, true);  // there is room again
       mtg_destroy(ctx);
     }
+    // A prompt that fails at its allocation number `have` launches nothing, and its repeat
+    // makes all the buffers that are missing, the failed one first.
+    int total = 0;
+    for (int have = -1; have < total; ++have) {  // -1: none fails, to count them
+      mtg_ctx* ctx = context(64);
+      std::vector<float> in((size_t)16 * kHidden);
+      int asked = 0;
+      f.malloc_fails = [&](size_t) { return asked++ == have; };
+      f.launches.clear();
+      const int rc = mtg_prefill(ctx, in.data(), 16, nullptr);
+      if (have < 0) total = asked;
+      expect(rc == (have < 0 ? MTG_OK : MTG_ERR_NOMEM), "prefill without allocation", have, rc);
+      expect(have < 0 || f.launches.empty(), "launches without allocation", have);
+      const int before = asked - (have >= 0);
+      asked = -1000;  // none fails
+      expect(mtg_prefill(ctx, in.data(), 16, nullptr) == MTG_OK, "prefill again", have);
+      expect(before + asked + 1000 == total, "buffers after the repeat", before + asked + 1000, total);
+      f.malloc_fails = nullptr;
+      mtg_destroy(ctx);
+    }
+    expect(total >= 7, "prefill buffers", total);
     std::printf("weights %d: %d failures\n", type, failures);
     mtg_synth_free(synth);
   }
