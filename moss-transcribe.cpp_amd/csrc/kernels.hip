@@ -958,7 +958,19 @@ bool launch_mul_mat(hipStream_t s, const uint8_t* w, int n, int k, const float* 
   // panels to a CU (K 4,096, 16 rows, N 16,384: 56 us against the general path's 47; 8
   // rows: 37 against 46; K 1,024, N 151,936, one row: 38 against 55).
   const bool split = tiles <= 1024 && (int64_t)tiles * T * k <= (1 << 25);
-  if (4 * lds > 150 * 1024 && tiles > 512) return false;
+  // A larger panel: a workgroup per tile, all of them on the chip at once (three, two or
+  // one to a CU). A second round of panels costs more than the launch it saves: K 5,120, 9
+  // rows, N 4,096 31 us against the general path's 43, N 6,144 48 against 44; K 8,704, 8
+  // rows, N 4,096 42 against 49, N 4,352 67 against 50; K 14,336, N 4,352, one row 65
+  // against 61. One or two short rows (the second term) are as fast or faster all the
+  // same: K 8,704, N 4,352, one row 45 against 50; K 11,264, N 8,192 55 against 55.
+  // Walking such panels leaves half of the CUs idle: K 7,168, N 8,192, 16 rows 84 against
+  // 49; K 9,216, 8 rows 80 against 51.
+  if (4 * lds > 150 * 1024) {
+    const int resident = (int)(160 * 1024 / (lds + (size_t)G * 4096));  // workgroups per CU
+    const bool fits = tiles <= 256 * resident || (G == 1 && (T + 4) * k <= 57000);
+    if (!split || tiles > 512 || !fits) return false;
+  }
   const dim3 grid((unsigned)(split ? tiles : std::min((tiles + 3) / 4, 1024)));
 #define MTG_MUL_MAT(G_, SPLIT_)                                                                                       \
   do {                                                                                                                \

@@ -52,8 +52,29 @@ static void overlap() {
   }
 }
 
+// Panels of which a CU holds three, two or one: the one-launch kernel as long as all
+// tiles' workgroups are on the chip at once, or for a few short rows.
+static void large_panels() {
+  const struct {
+    int k, n, T, route;
+  } cases[] = {{4160, 4096, 16, 1}, {4160, 4112, 16, 2}, {4096, 8192, 16, 1}, {5120, 4096, 9, 1},  {5120, 6144, 9, 2},
+               {7168, 4096, 16, 1}, {7168, 8192, 16, 2}, {7168, 8192, 8, 1},  {8640, 8192, 7, 1},  {8704, 4096, 8, 1},
+               {8704, 4112, 8, 2},  {9216, 8192, 8, 2},  {11264, 8192, 1, 1}, {12288, 8192, 1, 2}, {9216, 8192, 2, 1},
+               {10240, 8192, 2, 2}, {14336, 4096, 8, 1}, {14336, 4112, 1, 2}, {4288, 8208, 1, 2}};
+  for (const auto& c : cases) {
+    Matrix m(c.k, c.n);
+    std::vector<float> x((size_t)c.T * c.k + 4), y((size_t)c.T * c.n + 4);
+    float* xa = (float*)(((uintptr_t)x.data() + 15) & ~(uintptr_t)15);
+    float* ya = (float*)(((uintptr_t)y.data() + 15) & ~(uintptr_t)15);
+    const int r = route(m, xa, c.T, ya);
+    if (r != c.route) std::fprintf(stderr, "K %d N %d: ", c.k, c.n);
+    expect(r == c.route, "route of T", c.T, r);
+  }
+}
+
 int main() {
   overlap();
+  large_panels();
   std::printf("{\"record\": \"mulMatRoute\", \"failures\": %d}\n", failures);
   return failures ? 1 : 0;
 }

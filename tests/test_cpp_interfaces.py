@@ -41,7 +41,8 @@ def test_erf_polynomials_round_as_the_series():
 
 
 def test_product_alone_takes_the_kernels_it_may():
-    """csrc/kernels.hip launch_mul_mat on the fake HIP runtime: x and y that overlap."""
+    """csrc/kernels.hip launch_mul_mat on the fake HIP runtime: x and y that overlap,
+    panels of which a CU holds few."""
     rec = _run("test_mul_mat_route", 60)
     assert rec == {"record": "mulMatRoute", "failures": 0}
 

@@ -64,3 +64,21 @@ def test_mul_mat_over_its_own_input(k, n, T, y_at):
     got = buf.cpu().numpy()
     assert np.array_equal(got[yo:yo + T * n].reshape(T, n), ref)
     assert (got[:min(xo, yo)] == 7.0).all() and (got[max(xo + T * k, yo + T * n):] == 7.0).all()
+
+
+@pytest.mark.parametrize("k,n,T", [(4160, 4096, 16), (4160, 4112, 9), (8640, 8192, 1), (8704, 4112, 8), (8704, 8192, 1)])
+def test_mul_mat_large_panels(k, n, T):
+    """Both sides of the choice by the panels a CU holds (one, two; more tiles than that)."""
+    print("mul_mat, large panels: k %d n %d T %d" % (k, n, T), flush=True)
+    rng = np.random.default_rng(k + n + T)
+    w = (rng.standard_normal((n, k)) * 0.02).astype(np.float32)
+    raw = np.empty(n * (k // 32) * 34, np.uint8)
+    mtg.lib().mtg_quantize_q8_0_weight(mtg.ptr(w), n * k, mtg.ptr(raw))
+    x = rng.standard_normal((T, k)).astype(np.float32)
+    packed = ctypes.c_void_p()
+    assert mtg.lib().mtg_q8_pack(mtg.ptr(raw), k, n, ctypes.byref(packed)) == 0
+    xd, yd = torch.from_numpy(x).cuda(), torch.zeros(T, n, device="cuda")
+    rc = mtg.lib().mtg_q8_mul_mat_dev(packed, ctypes.c_void_p(xd.data_ptr()), T, ctypes.c_void_p(yd.data_ptr()))
+    mtg.lib().mtg_q8_free(packed)
+    assert rc == 0
+    assert np.array_equal(yd.cpu().numpy(), oracle_py.mul_mat(mtg.TYPE_Q8_0, raw, k, n, x))
