@@ -972,22 +972,18 @@ bool launch_mul_mat(hipStream_t s, const uint8_t* w, int n, int k, const float* 
     if (!split || tiles > 512 || !fits) return false;
   }
   const dim3 grid((unsigned)(split ? tiles : std::min((tiles + 3) / 4, 1024)));
-#define MTG_MUL_MAT(G_, SPLIT_)                                                                                       \
-  do {                                                                                                                \
-    if (lds + 8192 > 65536 && hipFuncSetAttribute((const void*)k_mul_mat<G_, SPLIT_>,                                 \
-                                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) \
-      return false;                                                                                                   \
-    hipLaunchKernelGGL((k_mul_mat<G_, SPLIT_>), grid, dim3(256), lds, s, w, n, bps, x, T, y);                         \
-  } while (0)
-  if (G == 1) {
-    if (split) MTG_MUL_MAT(1, true);
-    else MTG_MUL_MAT(1, false);
-  } else {
-    if (split) MTG_MUL_MAT(2, true);
-    else MTG_MUL_MAT(2, false);
-  }
-#undef MTG_MUL_MAT
-  return true;
+  // The kernel's LDS limit is one value for all threads, so every call sets the same one.
+  // What the runtime refuses is the general path's, with no error left for later checks.
+  auto launch = [&](const void* kernel) {
+    hipError_t e = hipSuccess;
+    if (lds + 8192 > 65536) e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, kMulMatLds);
+    void* args[] = {&w, &n, (void*)&bps, &x, &T, &y};
+    if (e == hipSuccess) e = hipLaunchKernel(kernel, grid, dim3(256), args, lds, s);
+    if (e != hipSuccess) (void)hipGetLastError();
+    return e == hipSuccess;
+  };
+  if (G == 1) return launch(split ? (const void*)k_mul_mat<1, true> : (const void*)k_mul_mat<1, false>);
+  return launch(split ? (const void*)k_mul_mat<2, true> : (const void*)k_mul_mat<2, false>);
 }
 
 void launch_gemm_store(hipStream_t s, int G, const StepDesc* desc, const uint8_t* w, int n, int k,

@@ -57,7 +57,7 @@ void launch_norm_quant(hipStream_t s, const StepDesc* desc, const float* src, in
                        const float* gain, float eps, Panel panel, float* normed_out);
 // y = x (T rows, q8_0 on the device) times a packed q8_0 matrix, one launch; false where
 // its LDS panel, the pointers' alignment (16 bytes) or an overlap of x and y does not
-// allow it.
+// allow it, or the runtime refuses the launch: nothing has run then.
 bool launch_mul_mat(hipStream_t s, const uint8_t* w, int n, int k, const float* x, int T, float* y);
 // out[t][n] = W . x[t] for all rows of a packed matrix (epilogue: store).
 void launch_gemm_store(hipStream_t s, int G, const StepDesc* desc, const uint8_t* w, int n, int k,

@@ -41,6 +41,7 @@ struct State {
   std::vector<Copy> copies;
   std::function<bool(size_t)> malloc_fails;     // by size
   std::function<bool(const std::string&)> launch_fails, attribute_fails;
+  std::function<void()> attribute_set;          // after an attribute is set
   int last_error = kOk;
   uintptr_t handles = 0;
 };
@@ -93,6 +94,7 @@ int hipFuncSetAttribute(const void* f, int, int value) {
   fake::State& s = fake::state();
   if (s.attribute_fails && s.attribute_fails(fake::name_of(f))) return fake::fail(fake::kInvalid);
   s.lds_limit[f] = value;
+  if (s.attribute_set) s.attribute_set();
   return fake::kOk;
 }
 int hipGetLastError() {

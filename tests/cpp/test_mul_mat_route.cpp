@@ -72,7 +72,43 @@ static void large_panels() {
   }
 }
 
+// The LDS limit of the kernel is one value per process: another thread's call between
+// this one's setting of it and its launch. A launch or an attribute that is refused
+// sends the call to the general path and leaves no error behind.
+static void limits() {
+  const int n = 32, T = 16;
+  Matrix large(7168, n), small(4160, n);
+  std::vector<float> x(T * 7168 + 4), y(T * n + 4), y2(T * n + 4);
+  auto at = [](std::vector<float>& v) { return (float*)(((uintptr_t)v.data() + 15) & ~(uintptr_t)15); };
+  fake::State& f = fake::state();
+  bool inside = false;
+  int other = -1;
+  f.attribute_set = [&] {
+    if (inside) return;
+    inside = true;
+    other = mtg_q8_mul_mat_dev(small.w, at(x), T, at(y2));
+  };
+  f.launches.clear();
+  expect(mtg_q8_mul_mat_dev(large.w, at(x), T, at(y)) == MTG_OK && other == MTG_OK, "two calls", other);
+  f.attribute_set = nullptr;
+  expect(inside && fake::count("k_mul_mat") == 2 && f.launches.size() == 2, "both launch", (long)f.launches.size());
+  expect(f.last_error == 0, "an error left behind", f.last_error);
+
+  f.launch_fails = [](const std::string& k) { return k.find("k_mul_mat") != std::string::npos; };
+  expect(route(large, at(x), T, at(y)) == 2, "a refused launch");
+  f.launch_fails = nullptr;
+  expect(f.last_error == 0, "a refused launch leaves an error", f.last_error);
+  f.attribute_fails = [](const std::string& k) { return k.find("k_mul_mat") != std::string::npos; };
+  expect(route(large, at(x), T, at(y)) == 2, "a refused attribute");
+  f.attribute_fails = nullptr;
+  expect(f.last_error == 0, "a refused attribute leaves an error", f.last_error);
+  f.last_error = 7;  // another call's, which this one does not report as its own
+  expect(route(large, at(x), T, at(y)) == 1, "another call's error");
+  f.last_error = 0;
+}
+
 int main() {
+  limits();
   overlap();
   large_panels();
   std::printf("{\"record\": \"mulMatRoute\", \"failures\": %d}\n", failures);
