@@ -136,13 +136,18 @@ enum { PF_STORE = 0, PF_RESID = 1, PF_SWIGLU = 2, PF_BIAS = 3, PF_BIAS_GELU = 4,
 typedef int v16i __attribute__((ext_vector_type(16)));
 
 // 16 (4) bytes per lane from memory to LDS at lds + 16 (4) * lane, counted in vmcnt.
-// lds is a byte address, uniform over the wave.
+// lds is a byte address, uniform over the wave. m0 is the compiler's own for indexed
+// access: named, so that no value of its is taken to outlive the statement (the warning
+// about a reserved register says that it is not saved around it, which nothing needs).
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
 __device__ __forceinline__ void lds_fill16(const void* src, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(lds) : "memory");
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(lds) : "memory", "m0");
 }
 __device__ __forceinline__ void lds_fill4(const void* src, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(src), "s"(lds) : "memory");
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(src), "s"(lds) : "memory", "m0");
 }
+#pragma clang diagnostic pop
 
 // One 64-element step in LDS: the codes of 4 weight units, then 4 parts x 64 rows x 16
 // bytes of the activation, the units' scales (4 x 32 f16), [parity][64 rows] f32 scales.

@@ -1,7 +1,9 @@
 """The reference-named C++ interface (include/mtg_reference.hpp) through the C++
 test drivers in tests/cpp, built by __graft_entry__.build()."""
+import glob
 import json
 import os
+import re
 import subprocess
 
 import pytest
@@ -52,3 +54,16 @@ def test_prompts_of_several_blocks_and_their_buffers():
     without memory for the second set of rows."""
     rec = _run("test_prefill_buffers", 60)
     assert rec == {"record": "prefillBuffers", "failures": 0}
+
+
+def test_inline_asm_names_the_registers_it_writes():
+    """m0 is the compiler's too (LDS addressing, indexed registers): an asm statement that
+    writes it has to list it as clobbered."""
+    found = 0
+    for path in glob.glob(os.path.join(os.path.dirname(HERE), "moss-transcribe.cpp_amd", "csrc", "*.h*")):
+        with open(path) as f:
+            for text in re.findall(r"\basm\b[^;]*;", f.read()):
+                if re.search(r"s_mov_b32 m0", text):
+                    found += 1
+                    assert re.search(r':[^:]*"m0"[^:]*\)\s*;$', text), (os.path.basename(path), text)
+    assert found
