@@ -20,12 +20,26 @@
 // A workgroup takes 2 query tiles of 16; its four waves take chunks c = wave mod 4.
 // Every chunk's (l_c, O_c) is computed independently; the running (L, O) travels
 // from wave to wave through LDS in chunk order (the merge is 1 / 16 of the work).
-// Two workgroups per CU, two waves per SIMD (head_dim 64: three).
-// Measured against two exact passes with K and V^T staged by the whole workgroup:
-// 1,600 rows, f32 cache 289 -> 205 us per layer (the MFMAs alone: 69 us; the rest is
-// the estimates' reads of K at the start, vector work and the uneven causal blocks);
-// 2,048 rows after 14,336, f16 cache 3.84 -> 2.6 ms (1.64 ms); the
+// Two workgroups per CU, two waves per SIMD (head_dim 64: three; the encoder's 24 layers
+// 7.29 -> 7.19 ms). With an f32 cache the 256 registers do not hold everything: 13 or 14
+// are spilled, of which a chunk reloads four; the encoder's form spills 10 of its 168, the
+// f16-cache forms none.
+// Measured (kernel trace) against two exact passes with K and V^T staged by the whole
+// workgroup: 1,600 rows, f32 cache 289 -> 203 us per layer (the MFMAs alone: 69 us; the
+// rest is the estimates' reads of K at the start, vector work and the uneven causal
+// blocks); 2,048 rows after 14,336, f16 cache 3.80 -> 2.73 ms, 2.59 to 3.11 (1.64 ms); the
 // encoder's 1,500 rows x 16 heads 202 -> 153 us (60 us).
+//
+// What a repeat costs: the workgroup's exact pass once more. On noise, at most 0.3 % of the
+// workgroups repeat; on constant, half constant and nearly constant prompts and mel chunks
+// 2.6 % with an f32 cache (whole prefills up to 7 % longer) and 0.1 % with an f16 one.
+// Where a head's keys score alike to within f16's resolution (rows equal to 3e-6 and every
+// rotation but the slowest taken out of the keys), 25 to 81 % repeat with an f32 cache:
+// 1,600 rows, 8 layers 7.4 -> 8.4 ms a prompt (two exact passes: 10.4), 8,000 rows, 4
+// layers 24.9 -> 34.8 (35.0), but 16,384 rows, 4 layers 59.5 -> 98.8 (82.8), the one kind of
+// input found on which two exact passes are faster. Giving a pass up at its first score
+// above M (maxima only from there on) made that 93.0 and 1,600 rows no faster, and the
+// registers it takes cost ordinary prompts of 16,384 rows 1.5 to 2.5 %.
 #pragma once
 
 #include <hip/hip_fp16.h>

@@ -162,6 +162,8 @@ struct PgStage {
 // 50 and 65). Per layer at 1,600 rows: q|k|v 63 -> 33 us, gate/up 95 -> 50, o 33 -> 25,
 // down 48 -> 37 (before: codes staged through registers, one barrier per step with its
 // loads just ahead, block-diagonal 16 x 16 MFMAs).
+// Four workgroups leave a wave 128 registers: enough but for GELU's doubles (<4, 4>: 9 of
+// the running totals are spilled, moved once per K-slice).
 template <int EPI, int ST>
 __global__ void __launch_bounds__(256, ST == 4 ? 4 : 2)
 k_pf_gemm(const uint8_t* __restrict__ w, const uint8_t* __restrict__ w2, int N, int K,

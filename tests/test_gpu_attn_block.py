@@ -43,6 +43,31 @@ def test_prefill_with_nearly_equal_scores(S, kv_type):
     model.close()
 
 
+@pytest.mark.parametrize("kv_type", [mtg.TYPE_F32, mtg.TYPE_F16], ids=["f32kv", "f16kv"])
+def test_repeats_equal_the_16_row_path(kv_type):
+    """Eight layers of 1,600 such rows: 4,982 of the 6,400 workgroups repeat their exact pass
+    with an f32 cache and 597 with an f16 one (of the prompts above 1 of 304 at most, whose
+    estimates differ from the scores by the order of the sums alone). Against the 16-row path,
+    which has no estimates."""
+    S, layers = 1600, 8
+    print("near ties: S=%d kv %d, %d layers" % (S, kv_type, layers), flush=True)
+    model = mtg.SynthModel(mtg.TYPE_F32, seed=15, std=0.02, n_layers=layers, vocab=256)
+    gain = np.zeros(128, np.float32)
+    gain[56:64] = gain[120:128] = 1.0
+    for l in range(layers):
+        ctypes.memmove(model.desc.contents.layers[l].attn_k_norm, gain.ctypes.data, gain.nbytes)
+    rows = np.tile(mtg.normal(16, 0, 1024) * np.float32(0.03), (S, 1))
+    rows = (rows + mtg.normal(17, 0, S * 1024).reshape(S, 1024) * np.float32(3e-6)).astype(np.float32)
+    a, b = mtg.Decoder(model, S + 8, kv_type), mtg.Decoder(model, S + 8, kv_type)
+    b.prefill_mode(False)
+    _same(a.prefill(rows), b.prefill(rows), "hidden rows")
+    for x, y in zip(a.kv_read(S), b.kv_read(S)):
+        _same(x, y, "cache")
+    a.close()
+    b.close()
+    model.close()
+
+
 @pytest.mark.parametrize("n_frames", [66, 512, 514, 1030])
 def test_encoder_with_nearly_equal_scores(n_frames):
     """33, 256, 257 and 515 rows of one row with small noise (no positional embedding)."""
