@@ -704,18 +704,20 @@ int Ctx::prefill_blocks(const float* embeds, int S, float* hidden_out) {
 // computes, the previous block's hidden rows come back and the next one's inputs go out.
 // Copies of pageable memory hold the host, so on one stream every block boundary left the
 // device idle for both (16,384 rows: about 7 of 65 ms). Without memory for the second set
-// of rows (16.8 MB) the blocks do run that way.
+// of rows (16.8 MB) the blocks do run that way. On one stream its own order is enough: the
+// events of two would cost a short prompt 3 to 12 us (q8_0, one row, 4 layers: 408 to 417
+// against 405).
 template <class Block>
 int Ctx::prefill_pipeline(const float* embeds, int S, float* hidden_out, Block&& block) {
   const int H = hp.hidden, R = kPfRows, nb = (S + R - 1) / R;
   int rc = MTG_OK;
   if (!ev_start && (rc = check(hipEventCreate(&ev_start), "event"))) return rc;
   if (!ev_stop && (rc = check(hipEventCreate(&ev_stop), "event"))) return rc;
-  for (int i = 0; i < 2; ++i) {
-    if (!pf.up[i] && (rc = check(hipEventCreateWithFlags(&pf.up[i], hipEventDisableTiming), "event"))) return rc;
-    if (!pf.done[i] && (rc = check(hipEventCreateWithFlags(&pf.done[i], hipEventDisableTiming), "event"))) return rc;
-  }
   if (nb > 1) {
+    for (int i = 0; i < 2; ++i) {
+      if (!pf.up[i] && (rc = check(hipEventCreateWithFlags(&pf.up[i], hipEventDisableTiming), "event"))) return rc;
+      if (!pf.done[i] && (rc = check(hipEventCreateWithFlags(&pf.done[i], hipEventDisableTiming), "event"))) return rc;
+    }
     if (!pf.copy && (rc = check(hipStreamCreateWithFlags(&pf.copy, hipStreamNonBlocking), "stream"))) return rc;
   }
   const bool overlap = nb > 1 && pf_buffer(pf.x2, (size_t)R * H) && pf_buffer(pf.hid2, (size_t)R * H);
@@ -725,10 +727,10 @@ int Ctx::prefill_pipeline(const float* embeds, int S, float* hidden_out, Block&&
   auto up = [&](int b) {
     const int e = check(hipMemcpyAsync(x[b & 1], embeds + (size_t)b * R * H, (size_t)rows(b) * H * 4,
                                        hipMemcpyHostToDevice, cs), "prompt rows");
-    return e ? e : check(hipEventRecord(pf.up[b & 1], cs), "event");
+    return e || !overlap ? e : check(hipEventRecord(pf.up[b & 1], cs), "event");
   };
   auto down = [&](int b) {  // block b is done: its hidden rows; its x may be written again
-    const int e = check(hipStreamWaitEvent(cs, pf.done[b & 1], 0), "event");
+    const int e = overlap ? check(hipStreamWaitEvent(cs, pf.done[b & 1], 0), "event") : MTG_OK;
     if (e || !hidden_out) return e;
     return check(hipMemcpyAsync(hidden_out + (size_t)b * R * H, hid[b & 1], (size_t)rows(b) * H * 4,
                                 hipMemcpyDeviceToHost, cs), "hidden rows");
@@ -737,17 +739,18 @@ int Ctx::prefill_pipeline(const float* embeds, int S, float* hidden_out, Block&&
   if (!rc) rc = up(0);
   for (int b = 0; b < nb && !rc; ++b) {
     // the inputs of block b are there, and the copy stream is past block b - 2's hidden rows
-    if ((rc = check(hipStreamWaitEvent(s, pf.up[b & 1], 0), "event"))) break;
+    if (overlap && (rc = check(hipStreamWaitEvent(s, pf.up[b & 1], 0), "event"))) break;
     block(b * R, rows(b), x[b & 1], hid[b & 1]);
     if ((rc = check(hipGetLastError(), "prefill launch"))) break;
-    if ((rc = check(hipEventRecord(pf.done[b & 1], s), "event"))) break;
+    if (overlap && (rc = check(hipEventRecord(pf.done[b & 1], s), "event"))) break;
     if (overlap ? b > 0 && (rc = down(b - 1)) : (rc = down(b))) break;
     if (b + 1 < nb) rc = up(b + 1);
   }
   if (!rc && overlap) rc = down(nb - 1);
   if (!rc) rc = check(hipEventRecord(ev_stop, cs), "event");
   // both streams are idle before the call returns, also after an error
-  const int e1 = check(hipStreamSynchronize(cs), "prefill"), e2 = check(hipStreamSynchronize(s), "prefill");
+  const int e1 = check(hipStreamSynchronize(s), "prefill");
+  const int e2 = overlap ? check(hipStreamSynchronize(cs), "prefill") : MTG_OK;
   if (rc || (rc = e1) || (rc = e2)) return rc;
   float ms = 0.0f;
   if ((rc = check(hipEventElapsedTime(&ms, ev_start, ev_stop), "event"))) return rc;

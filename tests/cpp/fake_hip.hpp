@@ -42,6 +42,7 @@ struct State {
   std::function<bool(size_t)> malloc_fails;     // by size
   std::function<bool(const std::string&)> launch_fails, attribute_fails;
   std::function<void()> attribute_set;          // after an attribute is set
+  int waits = 0, stream_syncs = 0;              // hipStreamWaitEvent, hipStreamSynchronize
   int last_error = kOk;
   uintptr_t handles = 0;
 };
@@ -144,8 +145,14 @@ int hipStreamCreateWithFlags(void** s, unsigned) {
   return fake::kOk;
 }
 int hipStreamDestroy(void*) { return fake::kOk; }
-int hipStreamSynchronize(void*) { return fake::kOk; }
-int hipStreamWaitEvent(void*, void*, unsigned) { return fake::kOk; }
+int hipStreamSynchronize(void*) {
+  ++fake::state().stream_syncs;
+  return fake::kOk;
+}
+int hipStreamWaitEvent(void*, void*, unsigned) {
+  ++fake::state().waits;
+  return fake::kOk;
+}
 int hipEventCreateWithFlags(void** e, unsigned) {
   *e = fake::handle();
   return fake::kOk;

@@ -26,7 +26,10 @@ static void prompt(mtg_ctx* ctx, int S, bool want_hidden, bool two_streams) {
   fake::State& f = fake::state();
   f.launches.clear();
   f.copies.clear();
+  f.waits = f.stream_syncs = 0;
   expect(mtg_prefill(ctx, in.data(), S, want_hidden ? out.data() : nullptr) == MTG_OK, "prefill", S, two_streams);
+  // one stream keeps its own order: no events to wait for, one wait for its end
+  if (!two_streams) expect(f.waits == 0 && f.stream_syncs == 1, "waits on one stream", f.waits, f.stream_syncs);
   size_t up = 0, down = 0;
   void* compute = f.launches.empty() ? nullptr : f.launches[0].stream;
   std::map<const void*, size_t> rows_in;  // device buffer -> the end of what it was last filled with
